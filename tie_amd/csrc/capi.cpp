@@ -388,7 +388,7 @@ static int create_layer(const tie_hip_layer_desc *ds, tie_hip_layer **out)
 	const size_t b_router = align256((size_t)E * d * 4), b_bias = align256((size_t)E * 4);
 	const size_t b_gate = align256(E * L.gate.expert_bytes), b_up = align256(E * L.up.expert_bytes),
 		     b_down = align256(E * L.down.expert_bytes);
-	// [router | router bias | selection bias | transposed router | gate | up | down]
+	// [router | router bias | selection bias | router in operand order | gate | up | down]
 	L.bytes = 2 * b_router + 2 * b_bias + b_gate + b_up + b_down;
 	rc = dev_malloc(&L.alloc, L.bytes, "layer weights");
 	if (rc) {
@@ -400,7 +400,7 @@ static int create_layer(const tie_hip_layer_desc *ds, tie_hip_layer **out)
 	L.bias = ds->router_bias ? (const float *)(base + b_router) : nullptr;
 	L.routing = ds->routing;
 	L.pbias = ds->probs_bias ? (const float *)(base + b_router + b_bias) : nullptr;
-	L.routerT = (const float *)(base + b_router + 2 * b_bias);
+	L.routerM = (const float *)(base + b_router + 2 * b_bias);
 	L.gate.data = base + 2 * b_router + 2 * b_bias;
 	L.up.data = L.gate.data + b_gate;
 	L.down.data = L.up.data + b_up;
@@ -416,7 +416,7 @@ static int create_layer(const tie_hip_layer_desc *ds, tie_hip_layer **out)
 	if (e == hipSuccess && ds->probs_bias)
 		e = hipMemcpyAsync((void *)L.pbias, ds->probs_bias, (size_t)E * 4, kind, g.stream);
 	if (e == hipSuccess)
-		e = launch_router_transpose(L, g.stream);
+		e = launch_router_order(L, g.stream);
 	struct Src {
 		const ExpertTensor *t;
 		const void *p;
@@ -543,12 +543,13 @@ static int forward(tie_hip_layer *layer, const float *x, int T, int k, float *ou
 		XConvArgs xc;
 		const bool xconv = router_converts_x(L, T) && L.gate.type != TIE_GGML_BF16 && mfma_f16_operands(L);
 		if (xconv) {
-			// the tiled logits kernel writes the f16 A operand and range flags
+			// the logits kernel writes the f16 A operand and the parts of the
+			// range flags (in the remainder plane, which only BF16 weights use)
 			xc.xa = ws.xb;
-			xc.flag = ws.tok_flag;
+			xc.part = reinterpret_cast<uint8_t *>(ws.xlo);
 		}
-		HIP_TRY(launch_router_logits(L, x, T, ws.logits, s, z, xc));
-		HIP_TRY(launch_route_bucket(L, x, T, k, ws, s, xconv));
+		HIP_TRY(launch_router_logits(L, x, T, ws.logits, s, z, xconv ? &xc : nullptr));
+		HIP_TRY(launch_route_bucket(L, x, T, k, ws, s, xconv ? &xc : nullptr));
 		prof_end(s);
 		if (!route_appends(T)) {
 			prof_begin("dispatch", s);

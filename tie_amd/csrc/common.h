@@ -93,7 +93,7 @@ __host__ __device__ inline size_t panel_bytes(int type)
 struct Layer {
 	int d = 0, F = 0, E = 0;
 	const float *router = nullptr; // [E][d]
-	const float *routerT = nullptr; // [d][E] (the tiled router kernel's layout)
+	const float *routerM = nullptr; // the same in router_mm_kernel's operand order (E a multiple of 16)
 	const float *bias = nullptr;   // [E] or null, added to the logits
 	int routing = 0;               // ROUTE_SOFTMAX (Qwen3) or ROUTE_SIGMOID (LFM2)
 	const float *pbias = nullptr;  // [E] or null: LFM2 selection bias (exp_probs_b_bias)
@@ -151,17 +151,20 @@ struct ZeroArgs {
 	int32_t *one = nullptr;
 };
 // The matrix-core path's f16 A operand of x (gate/up; K order 0,2,1,3,4,6,5,7
-// inside each group of 8) and the token's range flag (1: a value not finite
-// or not below 65504 in magnitude), written by the tiled logits kernel from
-// the x rows it stages anyway (router_converts_x); the routing kernel then
-// only lists the flagged tokens.
+// inside each group of 8), written by the matrix-core logits kernel from the
+// x rows it stages anyway (router_converts_x), each expert tile's workgroups
+// converting a share of K: part[t][tile] says whether the share holds a value
+// not finite or not below 65504 in magnitude.  The routing kernel ORs a
+// token's parts (tiles of them) into its range flag and lists the flagged
+// tokens.
 struct XConvArgs {
 	uint16_t *xa = nullptr;
-	int32_t *flag = nullptr;
+	uint8_t *part = nullptr;
+	int tiles = 0; // set by launch_router_logits
 };
 bool router_converts_x(const Layer &L, int T);
 hipError_t launch_router_logits(const Layer &L, const float *x, int T, float *logits, hipStream_t s,
-				ZeroArgs z = ZeroArgs(), XConvArgs xc = XConvArgs());
+				ZeroArgs z = ZeroArgs(), XConvArgs *conv = nullptr);
 // the matrix-core path's routing appends its pairs to the per-expert lists
 // (atomics on the counts) up to this many tokens; above, selection bytes
 // and bucket_plan (contended atomics: T=2048 35 us against 10 us)
@@ -182,16 +185,16 @@ inline bool route_appends(int T)
 #endif
 // the matrix-core path's selection, grouping into per-expert buckets and
 // A-operand conversion (mfma.hip)
-// converted: the logits kernel wrote the f16 A operand and the range flags
-// (XConvArgs); the routing then only lists the flagged tokens
+// conv (or null): the logits kernel wrote the f16 A operand and the parts of
+// the range flags; the routing then only lists the flagged tokens
 hipError_t launch_route_bucket(const Layer &L, const float *x, int T, int k, Workspace &ws, hipStream_t s,
-			       bool converted);
+			       const XConvArgs *conv);
 hipError_t launch_bucket_plan(const Layer &L, int T, int k, Workspace &ws, hipStream_t s);
 hipError_t launch_router_select(const Layer &L, int T, int k, const float *logits, int32_t *topk_idx, float *topk_w,
 				hipStream_t s);
 hipError_t launch_router(const Layer &L, const float *x, int T, int k, float *logits, int32_t *topk_idx,
 			 float *topk_w, hipStream_t s);
-hipError_t launch_router_transpose(const Layer &L, hipStream_t s);
+hipError_t launch_router_order(const Layer &L, hipStream_t s);
 hipError_t launch_dispatch(const Layer &L, int T, int k, const int32_t *topk_idx, Workspace &ws, hipStream_t s);
 hipError_t launch_route_group(const Layer &L, int T, int k, const float *logits, Workspace &ws, hipStream_t s);
 hipError_t launch_exact_block(const Layer &L, const float *x, int T, int k, const float *silu, Workspace &ws,

@@ -1712,7 +1712,8 @@ struct BucketArgs {
 	float *topk_w;
 	uint8_t *sel;
 	int32_t *cnt, *bucket; // non-null: append the pairs to the lists directly (small T)
-	int converted;         // MODE 1: the logits kernel wrote the A operand and flag[t] already
+	const uint8_t *part;   // MODE 1, non-null: the logits kernel wrote the A operand; [T][tiles] range flag parts
+	int tiles;
 	const float *x;
 	uint16_t *xa, *xlo;
 	int32_t *flag, *list, *count;
@@ -1755,7 +1756,7 @@ template <int MODE> __global__ __launch_bounds__(RB_THREADS) void route_bucket_k
 	const float4 *xr = reinterpret_cast<const float4 *>(r.x + (size_t)t * r.d);
 	const int n4 = r.d / 4;
 	float4 xv[RB_X];
-	const bool conv = !(MODE == 1 && r.converted);
+	const bool conv = !(MODE == 1 && r.part);
 	if (conv) {
 #pragma unroll
 		for (int i = 0; i < RB_X / 2; i++) {
@@ -1778,9 +1779,11 @@ template <int MODE> __global__ __launch_bounds__(RB_THREADS) void route_bucket_k
 	}
 	if constexpr (MODE == 1) {
 		if (!conv) {
-			// the A operand and the flag came with the logits: its sub-block
-			// sums from it, then list the token
+			// the A operand and the flag's parts came with the logits: its
+			// sub-block sums from it, then list the token
 			int sbad = 0;
+			for (int i = lane; i < r.tiles; i += 64)
+				sbad |= r.part[(size_t)t * r.tiles + i];
 			if (r.xsum) {
 				const int nsub = r.d / 32;
 				const f16x8 *xr8 = reinterpret_cast<const f16x8 *>(r.xa + (size_t)t * r.d);
@@ -1795,12 +1798,13 @@ template <int MODE> __global__ __launch_bounds__(RB_THREADS) void route_bucket_k
 					}
 					sbad |= store_xsum(r.xsum, t, nsub, g8 >> 2, part, g8 < r.d / 8);
 				}
-				sbad = __any(sbad);
 			}
-			if (lane == 0 && sbad && !r.flag[t])
-				r.flag[t] = 1;
-			if (lane == 0 && r.flag[t])
-				r.list[atomicAdd(r.count, 1)] = t;
+			sbad = __any(sbad);
+			if (lane == 0) {
+				r.flag[t] = sbad;
+				if (sbad)
+					r.list[atomicAdd(r.count, 1)] = t;
+			}
 			return;
 		}
 	}
@@ -1882,7 +1886,7 @@ static bool mfma_gu_qfold(const Layer &L, int npairs)
 }
 
 hipError_t launch_route_bucket(const Layer &L, const float *x, int T, int k, Workspace &ws, hipStream_t s,
-			       bool converted)
+			       const XConvArgs *conv)
 {
 	BucketArgs r;
 	r.logits = ws.logits;
@@ -1905,7 +1909,8 @@ hipError_t launch_route_bucket(const Layer &L, const float *x, int T, int k, Wor
 	r.flag = ws.tok_flag;
 	r.list = ws.fix_list;
 	r.count = ws.fix_count;
-	r.converted = converted && L.gate.type != TIE_GGML_BF16 && TIE_MFMA_F16;
+	r.part = conv ? conv->part : nullptr;
+	r.tiles = conv ? conv->tiles : 0;
 	r.xsum = mfma_gu_qfold(L, T * k) ? ws.xsum : nullptr;
 	const dim3 grid((T + RB_THREADS / 64 - 1) / (RB_THREADS / 64));
 	if (L.gate.type == TIE_GGML_BF16)

@@ -12,11 +12,10 @@
 // more than a launch on this multi-XCD part):
 //   router_small   T <= 4: one workgroup per expert row, row and tokens
 //                  staged in LDS, one thread per (token, lane) chain.
-//   router_mid     up to a few hundred tokens: one workgroup per (expert,
-//                  32 tokens), row in LDS, x streamed from L2.
-//   router_logits  large T: 32 tokens x 32 experts per workgroup over the
-//                  transposed router matrix staged by direct global->LDS
-//                  loads.
+//   router_mid     2 to 32 tokens (any number when E is not a multiple of
+//                  16): one workgroup per (expert, 16 or 32 tokens), row in
+//                  LDS, x streamed from L2.
+//   router_mm      more: the chains on the fp32 matrix cores.
 // Selection kernel: router_topk (a wave per token, E <= 1024).  Small
 // batches select
 // and group in one workgroup instead (route_group_kernel, dispatch.hip).
@@ -185,220 +184,267 @@ __global__ __launch_bounds__(TOK * 8) void router_mid_kernel(const float *__rest
 		logits[(size_t)t * E + e] = bias ? r + bias[e] : r;
 }
 
-// ------------------------------------------------------------ router_logits
-// One workgroup (8 waves) per RT_TOK tokens x 32 experts.  Thread (l, eg,
-// tg) runs the lane-l chains of experts 4eg..4eg+3 x tokens RT_TPT*tg..,
-// each in TIE's order (i ascending): per step one 16-byte LDS read of the 4
-// weights and RT_TPT reads of x feed 4*RT_TPT FMAs.  K advances RT_KC at a
-// time through a double-buffered LDS pipeline filled by direct global->LDS
-// loads (global_load_lds_dwordx4): the x rows as they are (token-major) and
-// the matching RT_KC rows x 32 experts of the transposed router matrix,
-// whose 16-byte column groups are XOR-swizzled by row (conflict-free
-// reads).  16 tokens and 128-wide K chunks keep the LDS at 48 KiB (three
-// workgroups per CU); 32 x 256 (128 KiB, one per CU) took 33 us at T = 512
-// against 26 us.
-#ifndef TIE_RT_TOK
-#define TIE_RT_TOK 16
-#endif
-#ifndef TIE_RT_KC
-#define TIE_RT_KC 128
-#endif
-constexpr int RT_TOK = TIE_RT_TOK, RT_EXP = 32, RT_KC = TIE_RT_KC, RT_THREADS = 512, RT_NW = RT_THREADS / 64;
-constexpr int RT_TPT = RT_TOK / 8;              // tokens per thread
-constexpr int RT_WBYTES = RT_KC * RT_EXP * 4;   // W^T chunk (16 KiB)
-constexpr int RT_XBYTES = RT_TOK * RT_KC * 4;   // x chunk (8 KiB)
-constexpr int RT_BUF = RT_WBYTES + RT_XBYTES;
-constexpr int RT_LDS = 2 * RT_BUF;              // double-buffered (48 KiB: three workgroups per CU)
-#ifndef TIE_RT_IB
-#define TIE_RT_IB 16
-#endif
-constexpr int RT_IB = TIE_RT_IB < RT_KC / 8 ? TIE_RT_IB : RT_KC / 8; // K steps whose operands are read ahead
-// the tiled kernel above this many tokens (below: router_mid)
-#ifndef TIE_RT_MIN_T
-#define TIE_RT_MIN_T 256
-#endif
+// ------------------------------------------------------------ router_mm
+// TIE's chains on the fp32 matrix cores.  v_mfma_f32_16x16x4_f32 computes
+// D[m][n] = fma(a[m][3], b[3][n], fma(a[m][2], b[2][n], fma(a[m][1], b[1][n],
+// fma(a[m][0], b[0][n], C[m][n])))) with every step rounded as v_fma_f32
+// rounds it (compared bit for bit over ordinary values, denormals,
+// infinities and NaN: 1.5 M results of each kind), so with K index kk =
+// step 4s + kk of chain l it is exactly 4 steps of TIE's lane-l accumulator
+// for 16 tokens x 16 experts, at twice the FMA rate of the vector unit and
+// a 16th of its operand reads per FMA.
+//
+// One workgroup (8 waves) per 16 NT tokens x 16 NE experts; wave w runs chain
+// l = w.  K advances RM_KC = 256 inputs (8 MFMAs per chain and 16 x 16 tile)
+// at a time: the x rows come in by coalesced 16-byte loads RM_PD chunks ahead
+// and are transposed through a double-buffered LDS tile to the operand order;
+// the weights are stored in operand order at layer creation
+// (launch_router_order) and go straight to registers, RM_PD chunks ahead too.
+// Operand order, for chain l and 16 steps: lane (kk = lane / 16, r = lane %
+// 16) holds steps 4c + kk, c = 0..3, of row r in one 16-byte word.
+//
+// Bound: the matrix pipe at large T (T d E FMAs at 32 per clock and SIMD: 6.8
+// us at 2048 x 2048 x 128; the kernel without its loads and LDS traffic took
+// 15 us there), else the latency of the launch and the first loads (about 4
+// us) and of the chunks.  Against the kernels it replaced (LDS-tiled vector
+// FMAs above 256 tokens, router_mid below; 30B shape, same box): T=64 7.7 ->
+// 6.9 us, T=101 11.5 -> 7.3, T=256 19.7 -> 7.0, T=500 17.9 -> 9.3, T=1024
+// 19.4 -> 12.5, T=2048 28.2 -> 19.4; 235B T=1024 35.0 -> 19.6.  Up to 32
+// tokens router_mid stays: T=32 6.3 us against 7.2, T=8 5.0 against 6.5.
+// Four waves of two chains each, and 3, 4 or 6 chunks ahead: within 3%.
+constexpr int RM_NW = 8, RM_PD = 2, RM_MIN_T = 32;
+constexpr int RM_KC = 256, RM_G = RM_KC / 128;
+// LDS strides of the x tile (floats): K group of 4 lanes' rows, 16-step
+// group, chain; the writes of a wave (32 steps of 2 chains) then fall in
+// distinct banks, two lanes a bank
+constexpr int RM_SK = 68, RM_SG = 4 * RM_SK, RM_SL = RM_G * RM_SG + 8, RM_BUF = 8 * RM_SL;
 
-// The LDS offset of a generic pointer into LDS: a flat LDS address is the
-// shared aperture's base in the high 32 bits and the offset in the low 32,
-// so truncation gives the offset (a cast to the LDS address space would add
-// a null-pointer test: a 64-bit compare and select per address).
-__device__ __forceinline__ uint32_t rt_lds_addr(const void *p)
+typedef float rm_f4 __attribute__((ext_vector_type(4)));
+
+// whether 4 consecutive x values leave the f16 range (XConvArgs)
+__device__ __forceinline__ int rm_bad(const float4 a)
 {
-	return (uint32_t)(uintptr_t)p;
-}
-
-// 16 bytes from global memory to LDS address lds + 16 * lane (inline asm:
-// the stage barrier, not the compiler, waits for it)
-__device__ __forceinline__ void rt_dma16(const void *g, uint32_t lds)
-{
-	asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds) : "memory", "m0");
-}
-
-// chunk kc of W^T (8 rows per wave instruction; slot s of row r holds
-// column group s ^ (r%8)) and of x (one 1 KiB token row per instruction)
-__device__ __forceinline__ void rt_dma_chunk(const float *__restrict__ x, const float *__restrict__ WT, int E, int d,
-					     int t0, int e0, int nt, int kc, uint8_t *buf)
-{
-	const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-#pragma unroll
-	for (int c = 0; c < RT_KC / 8 / RT_NW; c++) {
-		const int row0 = 8 * (RT_NW * c + w), row = row0 + (lane >> 3);
-		const int cg = (lane & 7) ^ (row & 7);
-		rt_dma16(WT + (size_t)(kc + row) * E + e0 + 4 * cg,
-			 __builtin_amdgcn_readfirstlane(rt_lds_addr(buf + row0 * RT_EXP * 4)));
-	}
-#pragma unroll
-	for (int c = 0; c < RT_TOK / RT_NW; c++) {
-		const int t = RT_NW * c + w;
-		if (t < nt && lane < RT_KC / 4)
-			rt_dma16(x + (size_t)(t0 + t) * d + kc + 4 * lane,
-				 __builtin_amdgcn_readfirstlane(rt_lds_addr(buf + RT_WBYTES + t * RT_KC * 4)));
-	}
-}
-
-__device__ __forceinline__ void rt_barrier()
-{
-	asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
-typedef _Float16 rt_f16x8 __attribute__((ext_vector_type(8)));
-
-// XConvArgs' conversion of the RT_TOK x RT_KC chunk staged at xs (token-major
-// rows of RT_KC floats), K offset kc: thread (t, q) of the first 16 RT_TOK
-// converts floats 8q .. 8q + 7 of token t; bad: its range flag so far
-__device__ __forceinline__ void rt_convert_chunk(const float *xs, const XConvArgs &xc, int t0, int nt, int d, int kc,
-						 int &bad)
-{
-	constexpr int QPT = RT_KC / 8; // threads per token
-	const int t = threadIdx.x / QPT, q = threadIdx.x % QPT;
-	if (t >= nt || threadIdx.x >= RT_TOK * QPT)
-		return;
-	const float4 a = *reinterpret_cast<const float4 *>(xs + t * RT_KC + 8 * q);
-	const float4 c = *reinterpret_cast<const float4 *>(xs + t * RT_KC + 8 * q + 4);
-	const float m = __builtin_fmaxf(__builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(a.x), __builtin_fabsf(a.y)),
-							__builtin_fmaxf(__builtin_fabsf(a.z), __builtin_fabsf(a.w))),
-					__builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(c.x), __builtin_fabsf(c.y)),
-							__builtin_fmaxf(__builtin_fabsf(c.z), __builtin_fabsf(c.w))));
+	const float m = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(a.x), __builtin_fabsf(a.y)),
+					__builtin_fmaxf(__builtin_fabsf(a.z), __builtin_fabsf(a.w)));
 	// fmax drops NaN: test the values themselves for NaN
-	const bool nan = a.x != a.x || a.y != a.y || a.z != a.z || a.w != a.w || c.x != c.x || c.y != c.y ||
-			 c.z != c.z || c.w != c.w;
-	bad |= (nan || !(m < 65504.0f)) ? 1 : 0;
-	const rt_f16x8 h = {(_Float16)a.x, (_Float16)a.z, (_Float16)a.y, (_Float16)a.w,
-			    (_Float16)c.x, (_Float16)c.z, (_Float16)c.y, (_Float16)c.w};
-	*reinterpret_cast<rt_f16x8 *>(xc.xa + (size_t)(t0 + t) * d + kc + 8 * q) = h;
+	const bool nan = a.x != a.x || a.y != a.y || a.z != a.z || a.w != a.w;
+	return (nan || !(m < 65504.0f)) ? 1 : 0;
 }
 
-__global__ __launch_bounds__(RT_THREADS) void router_logits_kernel(const float *__restrict__ x,
-								   const float *__restrict__ WT,
-								   const float *__restrict__ bias, int T, int d, int E,
-								   float *__restrict__ logits, ZeroArgs z, XConvArgs xc)
+template <int NE, int NT, bool CONV>
+__global__ __launch_bounds__(64 * RM_NW) __attribute__((amdgpu_waves_per_eu(2))) void
+router_mm_kernel(const float *__restrict__ x, const float *__restrict__ WM, const float *__restrict__ bias, int T, int d,
+		 int E, float *__restrict__ logits, int by_token, ZeroArgs z, XConvArgs xc)
 {
+	constexpr int NW = RM_NW, PD = RM_PD;
+	constexpr int TOK = 16 * NT;       // tokens per workgroup
+	constexpr int XR = TOK / NW;       // x rows per wave
+	constexpr int BUF = NT * RM_BUF;   // floats of one half of the x tile
 	zero_words(z);
-	extern __shared__ __attribute__((aligned(16))) uint8_t rt_lds[];
+	__shared__ __attribute__((aligned(16))) float xs[2 * BUF];
+	const int tid = threadIdx.x, lane = tid & 63;
+	const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+	// workgroups go round-robin over the 8 XCDs, each with its own L2:
+	// consecutive ids take different token tiles with the expert tiles of a
+	// token tile on one XCD (by_token: x is the larger operand), or
+	// different expert tiles
+	const int net = E / (16 * NE), ntt = (T + TOK - 1) / TOK;
+	int tt, et;
+	if (by_token) {
+		tt = (int)(blockIdx.x / (8 * net)) * 8 + (int)(blockIdx.x % 8);
+		et = (int)(blockIdx.x / 8) % net;
+		if (tt >= ntt)
+			return;
+	} else {
+		et = (int)blockIdx.x % net;
+		tt = (int)blockIdx.x / net;
+	}
+	const int t0 = tt * TOK, nt = min(TOK, T - t0);
+	const int nck = d / RM_KC;
 
-	const int tid = threadIdx.x;
-	const int l = tid & 7, eg = (tid >> 3) & 7, tg = tid >> 6;
-	const int t0 = blockIdx.x * RT_TOK, e0 = blockIdx.y * RT_EXP;
-	const int nt = min(RT_TOK, T - t0);
-	const int nkc = d / RT_KC;
-	// float index of experts 4eg.. in W^T row r: slot eg ^ (r%8), r % 8 == l
-	const int wcol = 4 * (eg ^ l);
-	const int xo = (RT_TPT * tg) * RT_KC + l;
+	// x: thread loads float4 c4 = lane of rows w + NW j (rows past the batch
+	// re-read the last one: their outputs are not stored), at 32-bit offsets
+	// from a wave-uniform base
+	const char *xbase = reinterpret_cast<const char *>(x + (size_t)t0 * d);
+	uint32_t xo[XR];
+#pragma unroll
+	for (int j = 0; j < XR; j++)
+		xo[j] = (uint32_t)(min(w + NW * j, nt - 1) * d * 4 + lane * 16);
+	// its place in the tile: chains 4 (lane % 2) + 0..3, step i = lane / 2
+	const int st = lane >> 1;
+	float *xw = xs + 4 * (lane & 1) * RM_SL + (st >> 4) * RM_SG + (st & 3) * RM_SK + ((st >> 2) & 3);
+	// weights: tile et, chain l, step group g: 64 lanes x 16 bytes
+	const uint32_t tile = (uint32_t)d * 64; // bytes of a tile (16 experts)
+	const char *wbase = reinterpret_cast<const char *>(WM) + (size_t)et * NE * tile + (size_t)w * (tile / 8);
+	const uint32_t wo = lane * 16;
 
-	float acc[RT_TPT][4];
+	float4 xv[PD][XR];
+	rm_f4 wv[PD][NE][RM_G];
+	auto load_x = [&](int ck, float4 (&v)[XR]) {
+		const char *b = xbase + min(ck, nck - 1) * (RM_KC * 4);
 #pragma unroll
-	for (int a = 0; a < RT_TPT; a++)
+		for (int j = 0; j < XR; j++)
+			v[j] = *reinterpret_cast<const float4 *>(b + xo[j]);
+	};
+	auto load_w = [&](int ck, rm_f4 (&v)[NE][RM_G]) {
+		const char *b = wbase + min(ck, nck - 1) * (RM_G * 1024);
 #pragma unroll
-		for (int b = 0; b < 4; b++)
-			acc[a][b] = 0.0f;
+		for (int n = 0; n < NE; n++)
+#pragma unroll
+			for (int g = 0; g < RM_G; g++)
+				v[n][g] = *reinterpret_cast<const rm_f4 *>(b + n * tile + g * 1024 + wo);
+	};
+#pragma unroll
+	for (int p = 0; p < PD; p++) {
+		load_x(p, xv[p]);
+		load_w(p, wv[p]);
+	}
+	rm_f4 acc[NT][NE];
+#pragma unroll
+	for (int m = 0; m < NT; m++)
+#pragma unroll
+		for (int n = 0; n < NE; n++)
+			acc[m][n] = rm_f4{0.0f, 0.0f, 0.0f, 0.0f};
+	int bad[XR] = {};
 
-	// the first expert tile's workgroups also convert their tokens' x rows
-	const bool conv = xc.xa && blockIdx.y == 0;
-	int bad = 0;
-
-	rt_dma_chunk(x, WT, E, d, t0, e0, nt, 0, rt_lds);
-	rt_barrier();
-	for (int c = 0; c < nkc; c++) {
-		if (c + 1 < nkc)
-			rt_dma_chunk(x, WT, E, d, t0, e0, nt, (c + 1) * RT_KC, rt_lds + ((c + 1) & 1) * RT_BUF);
-		const float *ws = reinterpret_cast<const float *>(rt_lds + (c & 1) * RT_BUF);
-		const float *xs = reinterpret_cast<const float *>(rt_lds + (c & 1) * RT_BUF + RT_WBYTES);
-		// before the FMAs: the stores have the chunk's FMAs to land before the
-		// stage barrier (which waits for every vector memory operation)
-		if (conv)
-			rt_convert_chunk(xs, xc, t0, nt, d, c * RT_KC, bad);
-		// operands of RT_IB K steps read into registers first (their LDS
-		// latencies overlap), then the FMAs in K order
-		for (int i0 = 0; i0 < RT_KC / 8; i0 += RT_IB) {
-			float4 w4[RT_IB];
-			float xv[RT_IB][RT_TPT];
+	const int kk = lane >> 4, r = lane & 15;
+	const float *rb = xs + w * RM_SL + kk * RM_SK + 4 * r;
+	rm_f4 a[NT][RM_G];
+	// element c of x row j out of its register into chunk ck's half of the tile
+	auto put = [&](int ck, int j, int c, const float4 &v) {
+		const int row = w + NW * j;
+		xw[(ck & 1) * BUF + (row >> 4) * RM_BUF + 4 * (row & 15) + c * RM_SL] = c == 0 ? v.x : c == 1 ? v.y : c == 2 ? v.z : v.w;
+	};
+	// a share of the chunks per expert tile goes to the f16 A operand too
+	auto convert = [&](int ck, const float4 (&v)[XR]) {
 #pragma unroll
-			for (int j = 0; j < RT_IB; j++) {
-				w4[j] = *reinterpret_cast<const float4 *>(ws + (8 * (i0 + j) + l) * RT_EXP + wcol);
-#pragma unroll
-				for (int a = 0; a < RT_TPT; a++)
-					xv[j][a] = xs[xo + a * RT_KC + 8 * (i0 + j)];
-			}
-#pragma unroll
-			for (int j = 0; j < RT_IB; j++) {
-#pragma unroll
-				for (int a = 0; a < RT_TPT; a++) {
-					acc[a][0] = __builtin_fmaf(xv[j][a], w4[j].x, acc[a][0]);
-					acc[a][1] = __builtin_fmaf(xv[j][a], w4[j].y, acc[a][1]);
-					acc[a][2] = __builtin_fmaf(xv[j][a], w4[j].z, acc[a][2]);
-					acc[a][3] = __builtin_fmaf(xv[j][a], w4[j].w, acc[a][3]);
-				}
-			}
+		for (int j = 0; j < XR; j++) {
+			typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+			const int row = w + NW * j;
+			bad[j] |= rm_bad(v[j]);
+			if (row < nt)
+				*reinterpret_cast<h4 *>(xc.xa + (size_t)(t0 + row) * d + ck * RM_KC + 4 * lane) =
+					h4{(_Float16)v[j].x, (_Float16)v[j].z, (_Float16)v[j].y, (_Float16)v[j].w};
 		}
-		rt_barrier();
-	}
-	if (conv) {
-		// a token's flag: the OR over its RT_KC / 8 threads (aligned lane groups)
-		constexpr int QPT = RT_KC / 8;
-		static_assert(64 % QPT == 0, "a token's threads in one wave");
-		const unsigned long long b = __ballot(bad);
-		const int lane = tid & 63, t = tid / QPT;
-		if (tid < RT_TOK * QPT && lane % QPT == 0 && t < nt)
-			xc.flag[t0 + t] = ((b >> lane) & ((1ull << QPT) - 1ull)) != 0 ? 1 : 0;
-	}
-
-	// hsum8 over the 8 lanes l of each chain group (math_avx2.c:14-21 order)
+	};
+	auto get = [&](int ck) {
 #pragma unroll
-	for (int a = 0; a < RT_TPT; a++) {
+		for (int m = 0; m < NT; m++)
 #pragma unroll
-		for (int b = 0; b < 4; b++) {
-			float r = hsum8_lanes(acc[a][b]);
-			const int t = RT_TPT * tg + a, e = e0 + 4 * eg + b;
-			if (l == 0 && t < nt) {
-				if (bias)
-					r = r + bias[e];
-				logits[(size_t)(t0 + t) * E + e] = r;
-			}
-		}
-	}
-}
-
-// W [E][d] -> W^T [d][E] (once, at layer creation)
-__global__ void transpose_kernel(const float *__restrict__ W, float *__restrict__ WT, int E, int d)
-{
-	__shared__ float tile[32][33];
-	const int bx = blockIdx.x * 32, by = blockIdx.y * 32; // bx: k, by: e
-	for (int i = threadIdx.y; i < 32; i += 8) {
-		const int e = by + i, kk = bx + threadIdx.x;
-		tile[i][threadIdx.x] = (e < E && kk < d) ? W[(size_t)e * d + kk] : 0.0f;
-	}
+			for (int g = 0; g < RM_G; g++)
+				a[m][g] = *reinterpret_cast<const rm_f4 *>(rb + (ck & 1) * BUF + m * RM_BUF + g * RM_SG);
+	};
+#pragma unroll
+	for (int j = 0; j < XR; j++)
+#pragma unroll
+		for (int c = 0; c < 4; c++)
+			put(0, j, c, xv[0][j]);
+	if (CONV && et == 0)
+		convert(0, xv[0]);
+	load_x(PD, xv[0]);
 	__syncthreads();
-	for (int i = threadIdx.y; i < 32; i += 8) {
-		const int kk = bx + i, e = by + threadIdx.x;
-		if (kk < d && e < E)
-			WT[(size_t)kk * E + e] = tile[threadIdx.x][i];
+	get(0);
+	// chunk ck (weights in slot p; p a constant after unrolling): its MFMAs,
+	// with the next chunk's writes to the other half of the tile and, into the
+	// freed registers, the loads of chunks ck + 1 + PD (x) and ck + PD
+	// (weights) issued one after each MFMA, under its 32 cycles.  The fences
+	// keep that order.
+	auto step = [&](int ck, int p, bool more) {
+		constexpr int M = 8 * NT * NE, W = 4 * XR;
+		const int pn = (p + 1) % PD;
+		if (CONV && (ck + 1) % net == et && ck + 1 < nck)
+			convert(ck + 1, xv[pn]);
+		const char *bx = xbase + min(ck + 1 + PD, nck - 1) * (RM_KC * 4);
+		const char *bw = wbase + min(ck + PD, nck - 1) * (RM_G * 1024) + wo;
+#pragma unroll
+		for (int u = 0; u < M; u++) {
+			const int n = u % NE, m = u / NE % NT, q = u / (NE * NT) % 4, g = u / (M / RM_G);
+			acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[m][g][q], wv[p][n][g][q], acc[m][n], 0, 0, 0);
+#pragma unroll
+			for (int i = u * W / M; i < (u + 1) * W / M; i++) {
+				// (past the last chunk: a copy nothing reads)
+				put(ck + 1, i / 4, i % 4, xv[pn][i / 4]);
+				if (more && i % 4 == 3)
+					xv[pn][i / 4] = *reinterpret_cast<const float4 *>(bx + xo[i / 4]);
+			}
+			__builtin_amdgcn_sched_barrier(0);
+			if (more && (u + 1) % (M / RM_G) == 0) {
+				// a step group's weights are used up
+#pragma unroll
+				for (int i = 0; i < NE; i++)
+					wv[p][i][g] = *reinterpret_cast<const rm_f4 *>(bw + i * tile + g * 1024);
+				__builtin_amdgcn_sched_barrier(0);
+			}
+		}
+		__syncthreads();
+		get(ck + 1);
+	};
+	int c0 = 0;
+	for (; c0 + PD <= nck; c0 += PD)
+#pragma unroll
+		for (int p = 0; p < PD; p++)
+			step(c0 + p, p, true);
+#pragma unroll
+	for (int p = 0; p < PD - 1; p++)
+		if (c0 + p < nck)
+			step(c0 + p, p, false);
+	if (CONV) {
+		// this expert tile's share of a token's flag: the OR over its wave's
+		// lanes (the routing kernel ORs the tiles')
+#pragma unroll
+		for (int j = 0; j < XR; j++) {
+			const int any = __any(bad[j]);
+			if (lane == 0 && w + NW * j < nt)
+				xc.part[(size_t)(t0 + w + NW * j) * net + et] = any ? 1 : 0;
+		}
+	}
+	// hsum8: s_m = v[m] + v[m + 4], (s0 + s1) + (s2 + s3) (math_avx2.c:14-21
+	// order), over the waves through LDS.  D layout: lane l, register i:
+	// token 4 (l / 16) + i, expert l % 16.
+	constexpr int OT = 16 * 17; // floats of one wave's 16 x 16 sums
+	static_assert(NT * NE * NW * OT <= 2 * BUF, "sums in the x tile");
+	__syncthreads();
+#pragma unroll
+	for (int m = 0; m < NT; m++)
+#pragma unroll
+		for (int n = 0; n < NE; n++)
+#pragma unroll
+			for (int i = 0; i < 4; i++)
+				xs[((m * NE + n) * NW + w) * OT + (4 * kk + i) * 17 + r] = acc[m][n][i];
+	__syncthreads();
+	for (int o = tid; o < TOK * 16 * NE; o += 64 * NW) {
+		const int c = o % (16 * NE), t = o / (16 * NE);
+		const float *q = xs + (((t >> 4) * NE + (c >> 4)) * NW) * OT + (t & 15) * 17 + (c & 15);
+		float s4[4];
+#pragma unroll
+		for (int m = 0; m < 4; m++)
+			s4[m] = q[m * OT] + q[(m + 4) * OT];
+		const float sum = (s4[0] + s4[1]) + (s4[2] + s4[3]);
+		const int e = et * 16 * NE + c;
+		if (t < nt)
+			logits[(size_t)(t0 + t) * E + e] = bias ? sum + bias[e] : sum;
 	}
 }
 
-hipError_t launch_router_transpose(const Layer &L, hipStream_t s)
+// W [E][d] -> the operand order of router_mm_kernel (once, at layer
+// creation; E a multiple of 16): [E / 16][chain 8][d / 128][lane 64][4]
+__global__ void router_order_kernel(const float *__restrict__ W, float *__restrict__ WM, int E, int d)
 {
-	tie_launch(transpose_kernel, dim3((L.d + 31) / 32, (L.E + 31) / 32), dim3(32, 8), 0, s, L.router,
-			   (float *)L.routerT, L.E, L.d);
+	const size_t n = (size_t)E * d, step = (size_t)gridDim.x * blockDim.x;
+	const int ng = d / 128;
+	for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += step) {
+		const int q = (int)(i & 3), lane = (int)(i >> 2) & 63;
+		const size_t u = i >> 8;
+		const int g = (int)(u % ng), l = (int)(u / ng) & 7, et = (int)(u / ng / 8);
+		WM[i] = W[(size_t)(16 * et + (lane & 15)) * d + 8 * (16 * g + 4 * q + (lane >> 4)) + l];
+	}
+}
+
+hipError_t launch_router_order(const Layer &L, hipStream_t s)
+{
+	if (L.E % 16)
+		return hipSuccess; // no operand order: the row kernels serve every T
+	tie_launch(router_order_kernel, dim3(256), dim3(256), 0, s, L.router, (float *)L.routerM, L.E, L.d);
 	return hipGetLastError();
 }
 
@@ -422,18 +468,21 @@ __global__ __launch_bounds__(RW_THREADS) void router_topk_kernel(const float *__
 			     pbias);
 }
 
-static bool router_tiled(const Layer &L, int T)
+static bool router_on_mm(const Layer &L, int T)
 {
-	return T > TIE_RT_MIN_T && L.E % RT_EXP == 0 && L.d % RT_KC == 0 && L.routerT;
+	return T > RM_MIN_T && L.E % 16 == 0 && L.routerM;
 }
 
 bool router_converts_x(const Layer &L, int T)
 {
-	return router_tiled(L, T);
+	// (up to 256 tokens the routing kernel, a wave per token, converts the rows
+	// under its selection; above, sharing it with the logits is faster: 30B
+	// T=2048 19.4 + 7.0 us against 17.1 + 10.4)
+	return T > 256 && router_on_mm(L, T);
 }
 
 hipError_t launch_router_logits(const Layer &L, const float *x, int T, float *logits, hipStream_t s, ZeroArgs z,
-				XConvArgs xc)
+				XConvArgs *conv)
 {
 	const int d = L.d, E = L.E;
 	if (T <= TIE_RS_MAX_T && sizeof(float) * (size_t)(8 * (d / 8 + 4)) * (1 + RS_TOK) <= 160 * 1024) {
@@ -442,19 +491,27 @@ hipError_t launch_router_logits(const Layer &L, const float *x, int T, float *lo
 				   logits, z);
 		return hipGetLastError();
 	}
-	// the tiled kernel above 256 tokens: below that its one chunk in flight
-	// per K step leaves it waiting on memory, and router_mid is faster
-	if (router_tiled(L, T)) {
-		static bool attr = false;
-		if (!attr) {
-			const hipError_t err = hipFuncSetAttribute((const void *)router_logits_kernel,
-								   hipFuncAttributeMaxDynamicSharedMemorySize, RT_LDS);
-			if (err != hipSuccess)
-				return err;
-			attr = true;
-		}
-		tie_launch(router_logits_kernel, dim3((T + RT_TOK - 1) / RT_TOK, E / RT_EXP), dim3(RT_THREADS),
-				   RT_LDS, s, x, L.routerT, L.bias, T, d, E, logits, z, xc);
+	if (router_on_mm(L, T)) {
+		auto go = [&](auto kern, int tok, int exp) {
+			const int ntt = (T + tok - 1) / tok, net = E / exp;
+			const int by_token = T >= 256 ? 1 : 0; // x the larger operand
+			if (conv)
+				conv->tiles = net;
+			tie_launch(kern, dim3(by_token ? (ntt + 7) / 8 * 8 * net : ntt * net), dim3(64 * RM_NW), 0, s, x,
+				   L.routerM, L.bias, T, d, E, logits, by_token, z, conv ? *conv : XConvArgs());
+		};
+		// larger tiles (fewer x transpositions and weight reads per MFMA) once
+		// they still cover most of the CUs: 30B T=500 (64 tiles of 32 x 32)
+		// 9.3 us with 16 x 16 tiles, 12.5 with 16 x 32, 16.9 with 32 x 32;
+		// T=1024 (128) 16.6 / 12.5 / 17.5; T=1500 (188) 18.8 with 16 x 32, 18.5
+		// with 32 x 32; T=2048 (256) 23.6 / 19.4
+		const int t32 = E % 32 == 0 ? (T + 31) / 32 * (E / 32) : 0;
+		if (t32 >= 192)
+			conv ? go(router_mm_kernel<2, 2, true>, 32, 32) : go(router_mm_kernel<2, 2, false>, 32, 32);
+		else if (t32 >= 96)
+			conv ? go(router_mm_kernel<2, 1, true>, 16, 32) : go(router_mm_kernel<2, 1, false>, 16, 32);
+		else
+			conv ? go(router_mm_kernel<1, 1, true>, 16, 16) : go(router_mm_kernel<1, 1, false>, 16, 16);
 		return hipGetLastError();
 	}
 	const bool u64 = d % 512 == 0;
