@@ -1,0 +1,45 @@
+"""Dense exact products of 5 and more tokens (the block dots on the fp32
+matrix cores), bit for bit against the oracle's rows: quads of tokens and
+their remainders, one and several groups, one super-block column and more
+than the workgroup's waves, both workgroup sizes, and inputs whose products
+reach zeros of both signs, denormals and infinities."""
+import numpy as np
+import pytest
+
+import tie_amd
+from conftest import bits
+from oracle import bind
+from tie_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def device():
+    import torch
+    assert torch.cuda.is_available(), "GPU test without a GPU"
+    tie_amd.init(0)
+    yield
+    tie_amd.shutdown()
+
+
+@pytest.mark.parametrize("wtype", [synth.Q4_K, synth.Q6_K])
+@pytest.mark.parametrize("rows,inn,T", [(64, 256, 5), (64, 512, 6), (128, 256, 7), (64, 768, 8), (64, 256, 9),
+                                        (64, 512, 11), (64, 2304, 13), (4096, 256, 34)])
+def test_dense_exact_groups(wtype, rows, inn, T):
+    import torch
+    rng = np.random.default_rng(17 + rows + inn + T + wtype)
+    w = synth.expert_tensor(rng, wtype, 1, rows, inn)
+    x = synth.make_input(18 + T, T, inn)
+    x[1] *= np.float32(1e-36)      # products in the denormals
+    x[2, ::3] = np.float32(-0.0)
+    x[3] *= np.float32(1e36)       # and past the largest value
+    m = tie_amd.Matrix(w, wtype, rows, inn)
+    out = torch.empty((T, rows), device="cuda")
+    m.mat_mat(torch.from_numpy(x).cuda(), T, out)
+    torch.cuda.synchronize()
+    got, ref = out.cpu().numpy(), bind.mat_mat(x, w, wtype, rows)
+    m.close()
+    nan = np.isnan(ref)
+    np.testing.assert_array_equal(np.isnan(got), nan)
+    np.testing.assert_array_equal(bits(got)[~nan], bits(ref)[~nan])

@@ -127,6 +127,8 @@ template <int PC> __device__ __forceinline__ void step_fence(float (&a0)[PC][8],
 constexpr int GU_WAVES = TIE_GU_WAVES;
 constexpr int GU_THREADS = 64 * GU_WAVES;
 constexpr int PG_MAX = 16;        // pairs per LDS group
+constexpr int MM_PAIRS = 8;       // pairs per block dot of the matrix-core instances
+constexpr int DENSE_GROUP = 8;    // tokens per group of a dense matrix product
 constexpr int PART_FLOATS = 16384; // LDS budget of the per-block partial dots (64 KiB)
 // Routing in the gate/up prologue up to this T (E <= 128).  Only one token:
 // for T = 2..8 every workgroup repeating the selection and grouping of all
@@ -402,6 +404,238 @@ __device__ __forceinline__ void block_dots(const Q6KStream &S, XP *const xs[PC],
 	}
 }
 
+// ------------------------------------------------------------ block dots on
+// the fp32 matrix cores, for 4 NQ input rows at once.
+// v_mfma_f32_4x4x1_16b_f32 rounds every element like v_fma_f32 (compared bit
+// for bit, denormals, infinities and NaN included).  With the A operand's
+// block n broadcast to all 16 blocks (cbsz = 4, abid = n) it is
+//   D[pair i][row] = fma(x_i, w_row, C[pair i][row])
+// for 4 pairs and the wave's 64 rows: lane = row holds w_row and the 4
+// pairs' accumulators of its row, and the x values of 16 inputs x 4 pairs
+// are one register (lane 4n + i: input n of pair i), loaded by coalesced
+// vector loads.  The same FMAs in the same order per accumulator as
+// block_dots; 4 FMAs cost one 4-cycle issue slot (9 cycles of the matrix
+// pipe) instead of four, and a weight is dequantised once for up to 8 pairs.
+// Used by the dense products of 5 and more tokens (groups of 8): Q4_K 4096 x
+// 2048, 32 tokens 18.9 -> 11.4 us (3.9 us of it the matrix pipe, the rest the
+// launch, the first loads and the row sums), 100 tokens 46.2 -> 35.7, 256
+// tokens 108 -> 76; Q6_K 32 tokens 27.0 -> 23.1, 100 tokens 107 -> 65; Q6_K
+// 151936 x 2048, 8 tokens 296 -> 186 us.  The experts of the small batches
+// that run here have 1 or 2 pairs each, where a quad would be mostly empty.
+// Requesting the whole block at once instead of a group ahead: no faster.
+typedef float mm_f4 __attribute__((ext_vector_type(4)));
+template <int N> using ic = std::integral_constant<int, N>;
+template <int B, int E, typename F> __device__ __forceinline__ void static_for(F f)
+{
+	if constexpr (B < E) {
+		f(ic<B>{});
+		static_for<B + 1, E>(f);
+	}
+}
+template <int ABID> __device__ __forceinline__ mm_f4 mm4(float x, float w, mm_f4 c)
+{
+	return __builtin_amdgcn_mfma_f32_4x4x1f32(x, w, c, 4, ABID, 0);
+}
+
+// xl: per quad, the lane's input pointer (pair lane % 4 of the quad, input
+// 4 (lane / 4) of the block): float4 j holds inputs 64 j + 4 n + c (block n,
+// component c).  out[q]: the block dots of quad q's 4 pairs.
+template <int NQ>
+__device__ __forceinline__ void block_dots_mm(const Q4KStream &S, const float *const xl[NQ], mm_f4 out[NQ])
+{
+	const uint4 c0 = ld(S.p);
+	uint4 cur[2] = {ld(S.p + 64), ld(S.p + 128)};
+	mm_f4 xc[NQ], acc[NQ][16];
+#pragma unroll
+	for (int q = 0; q < NQ; q++)
+		xc[q] = *reinterpret_cast<const mm_f4 *>(xl[q]);
+	const float d = half_bits_to_float(c0.x & 0xffffu);
+	const float dmin = half_bits_to_float(c0.x >> 16);
+	const uint32_t s[3] = {c0.y, c0.z, c0.w};
+#pragma unroll
+	for (int q = 0; q < NQ; q++)
+#pragma unroll
+		for (int m = 0; m < 16; m++)
+			acc[q][m] = mm_f4{0.0f, 0.0f, 0.0f, 0.0f};
+	static_for<0, 4>([&](auto gc) {
+		constexpr int g = decltype(gc)::value;
+		uint4 nxt[2];
+		mm_f4 xn[NQ];
+		if constexpr (g < 3) {
+			guint4 *p = S.p + 64 * (3 + 2 * g);
+			launder(p);
+			nxt[0] = ld(p);
+			nxt[1] = ld(p + 64);
+#pragma unroll
+			for (int q = 0; q < NQ; q++)
+				xn[q] = *reinterpret_cast<const mm_f4 *>(xl[q] + 64 * (g + 1));
+			__builtin_amdgcn_sched_barrier(0);
+		}
+		float D1, M1, D2, M2;
+		q4k_sub_scale(s, 2 * g, d, dmin, D1, M1);
+		q4k_sub_scale(s, 2 * g + 1, d, dmin, D2, M2);
+		static_for<0, 8>([&](auto sc) {
+			constexpr int ss = decltype(sc)::value, o = ss >> 2, h = ss & 3;
+			uint32_t w = word(cur[o], h);
+			asm volatile("" : "+v"(w));
+			uint32_t lo = w & 0x0f0f0f0fu, hi = (w >> 4) & 0x0f0f0f0fu;
+			asm volatile("" : "+v"(lo), "+v"(hi));
+			float wl[4], wh[4];
+#pragma unroll
+			for (int i = 0; i < 4; i++) {
+				wl[i] = __builtin_fmaf(ubyte(lo, i), D1, M1);
+				wh[i] = __builtin_fmaf(ubyte(hi, i), D2, M2);
+			}
+#pragma unroll
+			for (int q = 0; q < NQ; q++)
+#pragma unroll
+				for (int i = 0; i < 4; i++)
+					acc[q][4 * h + i] = mm4<4 * o + h>(xc[q][i], wl[i], acc[q][4 * h + i]);
+#pragma unroll
+			for (int q = 0; q < NQ; q++)
+#pragma unroll
+				for (int i = 0; i < 4; i++)
+					acc[q][4 * h + i] = mm4<8 + 4 * o + h>(xc[q][i], wh[i], acc[q][4 * h + i]);
+			if constexpr (ss & 1)
+				__builtin_amdgcn_sched_barrier(0);
+		});
+		if constexpr (g < 3) {
+			cur[0] = nxt[0];
+			cur[1] = nxt[1];
+#pragma unroll
+			for (int q = 0; q < NQ; q++)
+				xc[q] = xn[q];
+		}
+	});
+#pragma unroll
+	for (int q = 0; q < NQ; q++)
+#pragma unroll
+		for (int p = 0; p < 4; p++) {
+			float v[8];
+#pragma unroll
+			for (int l = 0; l < 8; l++)
+				v[l] = acc[q][l][p] + acc[q][l + 8][p];
+			out[q][p] = hsum8(v);
+		}
+}
+
+// Q6_K: TIE rounds the product (q - 32) x on its own, so the matrix cores
+// form the products (C = -0: p = fma(x, q, -0) is the rounded product, its
+// sign kept where it is zero) and the vector unit adds fma(d*sc, p, acc).
+template <int NQ>
+__device__ __forceinline__ void block_dots_mm(const Q6KStream &S, const float *const xl[NQ], mm_f4 out[NQ])
+{
+	const uint4 sc4 = ld(S.p + 64 * 12);
+	const float d = half_bits_to_float(*(const uint16_t *)S.dp);
+	auto quarter = [&](int qt, uint4 (&c)[3]) {
+		const int n = qt >> 1, hl = qt & 1;
+		guint4 *q = S.p + 64 * (4 * n + hl);
+		launder(q);
+		c[0] = ld(q);
+		c[1] = ld(q + 128);
+		c[2] = ld(q + 64 * (8 + 2 * n + hl) - 64 * (4 * n + hl));
+	};
+	auto sc = [&](int j) { return (float)(int8_t)((word(sc4, j >> 2) >> (8 * (j & 3))) & 0xffu); };
+	uint4 cur[3];
+	quarter(0, cur);
+	mm_f4 xc[NQ][2], acc[NQ][16];
+#pragma unroll
+	for (int q = 0; q < NQ; q++) {
+		xc[q][0] = *reinterpret_cast<const mm_f4 *>(xl[q]);
+		xc[q][1] = *reinterpret_cast<const mm_f4 *>(xl[q] + 64);
+#pragma unroll
+		for (int m = 0; m < 16; m++)
+			acc[q][m] = mm_f4{0.0f, 0.0f, 0.0f, 0.0f};
+	}
+	mm_f4 nz = {-0.0f, -0.0f, -0.0f, -0.0f};
+	asm volatile("" : "+v"(nz));
+	static_for<0, 4>([&](auto qc) {
+		constexpr int qt = decltype(qc)::value;
+		uint4 nxt[3];
+		if constexpr (qt < 3) {
+			quarter(qt + 1, nxt);
+			__builtin_amdgcn_sched_barrier(0);
+		}
+		static_for<0, 4>([&](auto stc) {
+			constexpr int st = 4 * qt + decltype(stc)::value;
+			constexpr int n = st >> 3, l = 8 * ((st >> 1) & 3), hw = st & 1, is = l >= 16 ? 1 : 0;
+			const float W[4] = {d * sc(8 * n + is + 0), d * sc(8 * n + is + 2), d * sc(8 * n + is + 4),
+					    d * sc(8 * n + is + 6)};
+			constexpr int dw = ((l & 8) >> 2) + hw;
+			uint32_t L = word(cur[0], dw), L2 = word(cur[1], dw), H = word(cur[2], dw);
+			asm volatile("" : "+v"(L), "+v"(L2), "+v"(H));
+			const uint32_t qb[4] = {q6_codes(L, 0, H, 0), q6_codes(L2, 0, H, 2), q6_codes(L, 4, H, 4),
+						q6_codes(L2, 4, H, 6)};
+			// runs 0, 64 feed accumulators m < 8 (TIE's a0), 32, 96 the others
+			static_for<0, 4>([&](auto rc) {
+				constexpr int r = decltype(rc)::value, a1 = r & 1;
+				uint32_t qw = qb[r];
+				asm volatile("" : "+v"(qw));
+				float f[4];
+#pragma unroll
+				for (int i = 0; i < 4; i++)
+					f[i] = sbyte_f(qw, i);
+#pragma unroll
+				for (int q = 0; q < NQ; q++) {
+					mm_f4 p[4];
+#pragma unroll
+					for (int i = 0; i < 4; i++)
+						p[i] = mm4<l / 4 + hw + 8 * a1>(xc[q][r >> 1][i], f[i], nz);
+#pragma unroll
+					for (int i = 0; i < 4; i++) {
+						mm_f4 &A = acc[q][8 * a1 + 4 * hw + i];
+#pragma unroll
+						for (int k = 0; k < 4; k++)
+							A[k] = __builtin_fmaf(W[r], p[i][k], A[k]);
+						asm volatile("" : "+v"(A)); // (keeps the FMAs here: see step_fence)
+					}
+				}
+			});
+		});
+		if constexpr (qt < 3) {
+#pragma unroll
+			for (int i = 0; i < 3; i++)
+				cur[i] = nxt[i];
+		}
+		if constexpr (qt == 1) {
+#pragma unroll
+			for (int q = 0; q < NQ; q++) {
+				xc[q][0] = *reinterpret_cast<const mm_f4 *>(xl[q] + 128);
+				xc[q][1] = *reinterpret_cast<const mm_f4 *>(xl[q] + 192);
+			}
+		}
+	});
+#pragma unroll
+	for (int q = 0; q < NQ; q++)
+#pragma unroll
+		for (int p = 0; p < 4; p++) {
+			float v[8];
+#pragma unroll
+			for (int l = 0; l < 8; l++)
+				v[l] = acc[q][l][p] + acc[q][l + 8][p];
+			out[q][p] = hsum8(v);
+		}
+}
+
+// The block dots of np <= 4 NQ pairs of a group on the matrix cores; xrow(q):
+// the block's inputs of pair q (per lane; pairs past np repeat the last)
+template <int NQ, typename Block, typename XF>
+__device__ __forceinline__ void pairs_mm(const Block &blk, int np, XF xrow, float *part_b, int lane)
+{
+	const float *xl[NQ];
+#pragma unroll
+	for (int q = 0; q < NQ; q++)
+		xl[q] = xrow(min(4 * q + (lane & 3), np - 1)) + 4 * (lane >> 2);
+	mm_f4 out[NQ];
+	block_dots_mm<NQ>(blk, xl, out);
+#pragma unroll
+	for (int q = 0; q < NQ; q++)
+#pragma unroll
+		for (int p = 0; p < 4; p++)
+			if (4 * q + p < np)
+				part_b[(4 * q + p) * 64 + lane] = out[q][p];
+}
+
 template <int TYPE> struct BlockOf;
 template <> struct BlockOf<TIE_GGML_Q4_K> {
 	using type = Q4KStream;
@@ -467,6 +701,7 @@ struct ExactArgs {
 	int32_t *offsets, *pairs, *active; // grouping (global)
 	int pg_cap;           // pairs per LDS group
 	int inline_route;
+	int dense;            // pairs are the tokens in order, slot s those from s * DENSE_GROUP on (no lists)
 	int single;           // T = 1 mode: slot j = pair j of expert topk_idx[j], no grouping
 	int routing;          // ROUTE_SOFTMAX / ROUTE_SIGMOID (inline routing)
 	const float *pbias;   // [E] selection bias of ROUTE_SIGMOID, or null
@@ -539,7 +774,7 @@ template <int TYPE, bool FUSED, int PM>
 __global__ __launch_bounds__(GU_THREADS) GU_OCC void exact_gu_kernel(ExactArgs a)
 {
 	// fused: as many waves as the launch chose; split: GU_WAVES
-	const int NW = FUSED ? __builtin_amdgcn_readfirstlane(blockDim.x >> 6) : GU_WAVES;
+	const int NW = FUSED || PM == MM_PAIRS ? __builtin_amdgcn_readfirstlane(blockDim.x >> 6) : GU_WAVES;
 	using Block = typename BlockOf<TYPE>::type;
 	extern __shared__ float part[]; // [mats][nb][pg_cap][64]
 	const int32_t *offsets = a.offsets, *pairs = a.pairs, *active = a.active;
@@ -565,6 +800,10 @@ __global__ __launch_bounds__(GU_THREADS) GU_OCC void exact_gu_kernel(ExactArgs a
 			return;
 		p0 = slot;
 		p1 = slot + 1;
+	} else if (PM == MM_PAIRS && a.dense) {
+		e = 0;
+		p0 = slot * DENSE_GROUP;
+		p1 = min(p0 + DENSE_GROUP, a.T);
 	} else {
 		if (slot >= active[a.E])
 			return;
@@ -596,16 +835,39 @@ __global__ __launch_bounds__(GU_THREADS) GU_OCC void exact_gu_kernel(ExactArgs a
 			Block blk;
 			load_block(panel_of(t), lane, blk);
 			auto xrow_b = [&](int q) {
-				const int pair = __builtin_amdgcn_readfirstlane(gp[q]);
+				const int pair = __builtin_amdgcn_readfirstlane(PM == MM_PAIRS && a.dense ? g0 + q : gp[q]);
 				return (cfloat *)(x + (size_t)(pair / k) * in + QK * b);
 			};
-			block_all_pairs<PM, Block, cfloat>(blk, np, xrow_b, part + (size_t)t * pg_cap * 64, lane);
+			if constexpr (PM == MM_PAIRS) {
+				auto xrow_v = [&](int q) {
+					return x + (size_t)(a.dense ? g0 + q : gp[q] / k) * in + QK * b;
+				};
+				float *part_t = part + (size_t)t * pg_cap * 64;
+				if constexpr (TYPE == TIE_GGML_Q4_K) {
+					if (np > 4)
+						pairs_mm<2>(blk, np, xrow_v, part_t, lane);
+					else
+						pairs_mm<1>(blk, np, xrow_v, part_t, lane);
+				} else {
+					// (8 pairs' accumulators and products do not fit the registers;
+					// a single pair is cheaper on the vector unit)
+					for (int q = 0; q < np; q += 4) {
+						if (np - q == 1)
+							pairs_chunk<1, Block, cfloat>(blk, q, xrow_b, part_t, lane);
+						else
+							pairs_mm<1>(blk, min(4, np - q), [&](int i) { return xrow_v(q + i); },
+								    part_t + q * 64, lane);
+					}
+				}
+			} else {
+				block_all_pairs<PM, Block, cfloat>(blk, np, xrow_b, part + (size_t)t * pg_cap * 64, lane);
+			}
 		}
 		__syncthreads();
 		// serial sums over super-blocks (math_avx2.c:762-766)
 		for (int i = threadIdx.x; i < np * 64; i += 64 * NW) {
 			const int q = i >> 6, r = i & 63;
-			const size_t o = (size_t)gp[q] * a.rows + rt * PANEL_ROWS + r;
+			const size_t o = (size_t)(PM == MM_PAIRS && a.dense ? g0 + q : gp[q]) * a.rows + rt * PANEL_ROWS + r;
 			float s0 = 0.0f;
 			for (int b = 0; b < nb; b++)
 				s0 = s0 + part[((size_t)b * pg_cap + q) * 64 + r];
@@ -900,7 +1162,7 @@ static int expected_active(int E, int k, int T, int max_active)
 // gate/up of one quantised type; fused (both matrices, h out) or one
 // matrix per blockIdx.z (row sums out)
 static hipError_t launch_gu_q(int type, bool fused, int nmat, int rows, int in, int max_active, ExactArgs g,
-			      hipStream_t s)
+			      hipStream_t s, bool mm = false)
 {
 	const int nb = in / QK;
 	const int mats = fused ? 2 : 1;
@@ -930,6 +1192,18 @@ static hipError_t launch_gu_q(int type, bool fused, int nmat, int rows, int in, 
 		block.x = 64 * pick_waves(fn, lds, (rows / PANEL_ROWS) * expected_active(g.E, g.k, g.T, max_active),
 					  2 * nb);
 	}
+	if (mm) {
+		// 8 waves (one workgroup per CU by registers) while one round of
+		// workgroups covers the grid, else 4 (two per CU: one's loads and
+		// sums overlap the other's dots; Q4_K 4096 x 2048, 8 / 4 waves: 32
+		// tokens 11.4 / 13.1 us, 100 tokens 39.7 / 35.7, 256 85 / 76; Q6_K
+		// 100 tokens 78 / 65)
+		const int w = (int)(grid.x * grid.y) > 256 ? 4 : 8;
+		block.x = 64 * (nb < w ? nb : w);
+	}
+	if (mm)
+		return type == TIE_GGML_Q4_K ? launch_q(exact_gu_kernel<TIE_GGML_Q4_K, false, MM_PAIRS>, grid, block, lds, st, s, g)
+					     : launch_q(exact_gu_kernel<TIE_GGML_Q6_K, false, MM_PAIRS>, grid, block, lds, st, s, g);
 	if (type == TIE_GGML_Q4_K)
 		return fused ? launch_q(exact_gu_kernel<TIE_GGML_Q4_K, true, PM>, grid, block, lds, st, s, g)
 			     : launch_q(exact_gu_kernel<TIE_GGML_Q4_K, false, PM>, grid, block, lds, st, s, g);
@@ -1117,8 +1391,6 @@ hipError_t launch_exact_block(const Layer &L, const float *x, int T, int k, cons
 // stride 0 (every group reads the one matrix), so groups spread over the
 // grid's y dimension and each workgroup computes one 64-row panel for one
 // group.  out[t][r], [T][rows].
-constexpr int DENSE_GROUP = 8;
-
 __global__ void dense_groups_kernel(int T, int G, int32_t *offsets, int32_t *pairs, int32_t *active)
 {
 	const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1140,12 +1412,6 @@ hipError_t launch_dense(const ExpertTensor &W, const float *x, int T, float *out
 	if (T == 0)
 		return hipSuccess;
 	const int G = dense_groups(T);
-	tie_launch(dense_groups_kernel, dim3((T + 1 + 255) / 256 > (G + 1 + 255) / 256 ? (T + 1 + 255) / 256
-											  : (G + 1 + 255) / 256),
-			   dim3(256), 0, s, T, G, ws.offsets, ws.pairs, ws.active);
-	hipError_t err = hipGetLastError();
-	if (err != hipSuccess)
-		return err;
 	ExactArgs a;
 	memset(&a, 0, sizeof a);
 	a.w[0] = W.data;
@@ -1161,10 +1427,13 @@ hipError_t launch_dense(const ExpertTensor &W, const float *x, int T, float *out
 	a.rows = W.rows;
 	a.in = W.in;
 	if (W.type == TIE_GGML_BF16) {
+		tie_launch(dense_groups_kernel, dim3((T + 1 + 255) / 256), dim3(256), 0, s, T, G, ws.offsets, ws.pairs,
+			   ws.active);
 		tie_launch(exact_gu_bf16_kernel, dim3(W.rows / PANEL_ROWS, G, 1), dim3(BF_THREADS), 0, s, a);
 		return hipGetLastError();
 	}
-	return launch_gu_q(W.type, false, 1, W.rows, W.in, G, a, s);
+	a.dense = 1;
+	return launch_gu_q(W.type, false, 1, W.rows, W.in, G, a, s, true);
 }
 
 } // namespace tie
