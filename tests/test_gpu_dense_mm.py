@@ -1,14 +1,17 @@
-"""Dense exact products of 5 and more tokens (the block dots on the fp32
+"""Dense products.  Exact ones of 5 and more tokens (the block dots on the fp32
 matrix cores), bit for bit against the oracle's rows: quads of tokens and
 their remainders, one and several groups, one super-block column and more
 than the workgroup's waves, both workgroup sizes, and inputs whose products
-reach zeros of both signs, denormals and infinities."""
+reach zeros of both signs, denormals and infinities.  Matrix-core ones on
+both sides of the K split and of each of its tile heights, down to one K
+stage per group, against a float64 model of their operands."""
 import numpy as np
 import pytest
 
 import tie_amd
 from conftest import bits
 from oracle import bind
+from test_gpu_mfma import MODEL_RL2, expert_weights, f16, rel_l2
 from tie_amd import synth
 
 pytestmark = pytest.mark.gpu
@@ -43,3 +46,22 @@ def test_dense_exact_groups(wtype, rows, inn, T):
     nan = np.isnan(ref)
     np.testing.assert_array_equal(np.isnan(got), nan)
     np.testing.assert_array_equal(bits(got)[~nan], bits(ref)[~nan])
+
+
+# one workgroup per CU or fewer (32-, 64- and 128-row tiles with their K
+# groups; 4 stages of 64 in all, then an odd number per block), and more
+@pytest.mark.parametrize("wtype", [synth.Q4_K, synth.Q6_K])
+@pytest.mark.parametrize("rows,inn,T", [(256, 256, 1), (512, 768, 33), (4096, 256, 512), (4096, 256, 1021),
+                                        (4096, 512, 2047), (4096, 256, 2049)])
+def test_dense_mfma_k_groups(wtype, rows, inn, T):
+    import torch
+    rng = np.random.default_rng(29 + rows + inn + T + wtype)
+    w = synth.expert_tensor(rng, wtype, 1, rows, inn)
+    x = synth.make_input(30 + T, T, inn)
+    m = tie_amd.Matrix(w, wtype, rows, inn)
+    out = torch.full((T, rows), np.nan, device="cuda")
+    m.mat_mat(torch.from_numpy(x).cuda(), T, out, flags=tie_amd.PATH_MFMA)
+    torch.cuda.synchronize()
+    m.close()
+    ref = f16(x).astype(np.float64) @ expert_weights(w, wtype, 0, rows, inn, True).astype(np.float64).T
+    assert rel_l2(out.cpu().numpy(), ref) <= MODEL_RL2

@@ -175,6 +175,13 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 #ifndef TIE_MFMA_DN_WPE
 #define TIE_MFMA_DN_WPE 2
 #endif
+// Kernel shape code of the dense products (or-ed with the tile rows): the K
+// stages split over n groups of 4 waves in one workgroup, each group with its
+// own stage buffers and accumulators, added up in LDS before the epilogue
+constexpr int mfma_ks(int n)
+{
+	return n << 10;
+}
 constexpr int NWAVES = 4;
 constexpr int MF_THREADS = 64 * NWAVES;
 constexpr int GU_COLS = 32 * NWAVES; // gate/up: F columns per tile (128)
@@ -218,6 +225,7 @@ struct MfmaArgs {
 				 // (y_shift only for f16 y)
 	float *y;                // down out, fp32 rows: y [pair][d] (BF16 experts), out [token][rows] (dense matrices)
 	uint16_t *y16;           // down out (quantised experts): y [pair][d] as f16(y 2^-y_shift)
+	int dense_t;             // K-split kernels: the tokens of the dense product
 	int mt_cap;              // pair rows per tile at most, below MT (0: MT; dense matrices at small T)
 	int direct;              // 32-row tiles, T <= MFMA_DIRECT_T: item (expert, slab), h rows [E][MFMA_DIRECT_T]
 	int32_t *tok_flag;       // [T] gate/up, h_f16: tokens whose h left the f16 range
@@ -237,7 +245,8 @@ __device__ __forceinline__ void flag_token(int32_t *flag, int32_t *list, int32_t
 
 template <int TYPE, bool DOWN = false, int MTR = 0> struct Cfg {
 	// pair rows per work tile at most (MTR: the small-tile gate/up kernel's)
-	static constexpr int MT = MTR                    ? MTR
+	static constexpr int KS = MTR >> 10 ? MTR >> 10 : 1; // K groups
+	static constexpr int MT = MTR                    ? (MTR & 1023)
 				  : TYPE == TIE_GGML_BF16 ? (DOWN ? MFMA_MT_DN_BF16 : MFMA_MT_GU_BF16)
 				  : DOWN                  ? MFMA_MT_DN
 							  : MFMA_MT_GU;
@@ -275,7 +284,8 @@ template <int TYPE, bool DOWN = false, int MTR = 0> struct Cfg {
 	// where they fit the budget of two workgroups per CU, else two
 	// workgroups per CU: the tiny-tile kernels TIE_MFMA_TINY_GU_WPC /
 	// _DN_WPC, the small-tile gate/up kernels 3, the others 2
-	static constexpr int WG_PER_CU = MTR == MFMA_MT_TINY ? (DOWN ? TIE_MFMA_TINY_DN_WPC : TIE_MFMA_TINY_GU_WPC)
+	static constexpr int WG_PER_CU = KS > 1                ? 1
+					 : MTR == MFMA_MT_TINY ? (DOWN ? TIE_MFMA_TINY_DN_WPC : TIE_MFMA_TINY_GU_WPC)
 					 : MTR && !DOWN ? 3
 					 : DOWN         ? TIE_MFMA_DN_WPE
 							: TIE_MFMA_GU_WPE;
@@ -285,6 +295,7 @@ template <int TYPE, bool DOWN = false, int MTR = 0> struct Cfg {
 	// many as the LDS budget of WG_PER_CU workgroups per CU allows, up to 4
 	// (quantised weights; BF16 weights go to registers: 2 activation buffers)
 	static constexpr int NS = !B_LDS ? 2
+				  : KS > 1 ? ((LDS_BUDGET - ROFF_BYTES) / KS / (ABUF + BBUF) < 4 ? (LDS_BUDGET - ROFF_BYTES) / KS / (ABUF + BBUF) : 4)
 				  : 4 * (ABUF + BBUF) + ROFF_BYTES <= LDS_BUDGET ? 4
 				  : 3 * (ABUF + BBUF) + ROFF_BYTES <= LDS_BUDGET ? 3 : 2;
 	static_assert(NWAVES == 4, "epilogue tile size");
@@ -299,7 +310,11 @@ template <int TYPE, bool DOWN = false, int MTR = 0> struct Cfg {
 	static constexpr bool SILU_LDS = !DOWN && !(MTR == MFMA_MT_TINY && TIE_TINY_SILU_GLOBAL);
 	static constexpr int EPI_BYTES =
 		(F16 && !SPLIT) ? (SILU_LDS ? 32768 : 0) + NWAVES * 16 * (DOWN ? 72 : 40) * 4 : 0;
-	static constexpr int STAGE_BYTES = LDS_A + LDS_B > EPI_BYTES ? LDS_A + LDS_B : EPI_BYTES;
+	static constexpr int RED_BYTES = (KS - 1) * MT * 64 * NWAVES * 4; // the K groups' accumulators
+	static constexpr int GRP_BYTES = LDS_A + LDS_B;
+	static constexpr int max2(int x, int y) { return x > y ? x : y; }
+	static constexpr int STAGE_BYTES = max2(max2(KS * GRP_BYTES, RED_BYTES), EPI_BYTES);
+	static_assert(KS == 1 || (NS >= 2 && STAGE_BYTES + ROFF_BYTES <= LDS_BUDGET), "K groups' LDS");
 	// The slot of 16-byte chunk c of row r is c ^ swz(r): the rows of a
 	// fragment read then spread over all LDS banks without row padding
 	// (which the direct global->LDS loads cannot make).
@@ -865,6 +880,18 @@ template <int N> __device__ __forceinline__ void stage_barrier_keep()
 	__builtin_amdgcn_s_barrier();
 }
 
+// The stage barrier that leaves the youngest `keep` <= K stages of PER loads
+// each in flight
+template <int K, int PER> __device__ __forceinline__ void stage_barrier_n(int keep)
+{
+	if constexpr (K <= 0)
+		stage_barrier();
+	else if (keep >= K)
+		stage_barrier_keep<K * PER>();
+	else
+		stage_barrier_n<K - 1, PER>(keep);
+}
+
 // Operand arithmetic of a quantised kernel: bf16 fragments, or f16 ones
 // (Q4_K gate/up).
 template <int TYPE, bool DOWN, int MTR = 0, bool F16 = Cfg<TYPE, DOWN>::F16> struct Ops;
@@ -976,8 +1003,13 @@ __device__ __forceinline__ void run_tile(const MfmaArgs &a, uint8_t *As, uint32_
 					 int pbase, int nrows, int slab, int pair_id)
 {
 	using C = Cfg<TYPE, DOWN, MTR>;
-	const int nk = a.in / C::KST;
-	const int t = threadIdx.x;
+	constexpr int KS = C::KS;
+	const int nk = a.in / C::KST / KS; // this K group's stages, from k0 on
+	const int t = KS > 1 ? threadIdx.x % MF_THREADS : threadIdx.x;
+	const int kg = KS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / MF_THREADS) : 0;
+	const int k0 = kg * nk;
+	uint8_t *const As0 = As;
+	As += kg * C::GRP_BYTES;
 #ifdef TIE_MFMA_TRACE
 	const unsigned long long t_start = __builtin_readcyclecounter();
 	unsigned long long t_loop = 0, bw_total = 0;
@@ -1064,8 +1096,8 @@ __device__ __forceinline__ void run_tile(const MfmaArgs &a, uint8_t *As, uint32_
 		// stage st's activations and weights into buffers st % NS
 		auto issue = [&](int st) {
 			if (st < nk) {
-				dma_a<TYPE, DOWN, NMT, MTR>(as, st, w, abuf(st));
-				dma_b<TYPE, DOWN, MTR>(bd, slab, st, w, bbuf(st));
+				dma_a<TYPE, DOWN, NMT, MTR>(as, k0 + st, w, abuf(st));
+				dma_b<TYPE, DOWN, MTR>(bd, slab, k0 + st, w, bbuf(st));
 			}
 		};
 		// direct loads one wave issues per stage (dma_a + dma_b)
@@ -1082,13 +1114,7 @@ __device__ __forceinline__ void run_tile(const MfmaArgs &a, uint8_t *As, uint32_
 #ifdef TIE_MFMA_TRACE
 			const unsigned long long tb = __builtin_readcyclecounter();
 #endif
-			const int keep = min(NS - 2, nk - 2 - st);
-			if (NS >= 4 && keep >= 2)
-				stage_barrier_keep<(NS >= 4 ? 2 * PER : 0)>();
-			else if (NS >= 3 && keep >= 1)
-				stage_barrier_keep<(NS >= 3 ? PER : 0)>();
-			else
-				stage_barrier();
+			stage_barrier_n<NS - 2, PER>(min(NS - 2, nk - 2 - st));
 #ifdef TIE_MFMA_TRACE
 			bwait += __builtin_readcyclecounter() - tb;
 #endif
@@ -1112,8 +1138,8 @@ __device__ __forceinline__ void run_tile(const MfmaArgs &a, uint8_t *As, uint32_
 		auto prep = [&](int st, int s, int slot) {
 			read(st, s, fa[slot]);
 			if (s == 0 || (TYPE == TIE_GGML_Q4_K && s % 4 == 0))
-				O::factors(b, st, s / 4, f);
-			O::template deq<DF || QF>(b, f, kc, st, s, fb[slot]);
+				O::factors(b, k0 + st, s / 4, f);
+			O::template deq<DF || QF>(b, f, kc, k0 + st, s, fb[slot]);
 		};
 		auto mm = [&](int slot) {
 #pragma unroll
@@ -1162,7 +1188,7 @@ __device__ __forceinline__ void run_tile(const MfmaArgs &a, uint8_t *As, uint32_
 				for (int sb = 0; sb < C::SPB; sb++) {
 					const int st = st0 + sb;
 					issue(st + NS - 1);
-					lds_b<TYPE, MTR>(bbuf(st), bp, bi, st, h, b);
+					lds_b<TYPE, MTR>(bbuf(st), bp, bi, k0 + st, h, b);
 					prep(st, 0, 0);
 #pragma unroll
 					for (int s = 0; s < C::NSTEP; s++) {
@@ -1201,7 +1227,7 @@ __device__ __forceinline__ void run_tile(const MfmaArgs &a, uint8_t *As, uint32_
 			// st + NS - 1 first, then its weights from LDS, then the steps)
 			for (int st = 0; st < nk; st++) {
 				issue(st + NS - 1);
-				lds_b<TYPE, MTR>(bbuf(st), bp, bi, st, h, b);
+				lds_b<TYPE, MTR>(bbuf(st), bp, bi, k0 + st, h, b);
 				prep(st, 0, 0);
 #pragma unroll
 				for (int s = 0; s < C::NSTEP; s++) {
@@ -1213,14 +1239,14 @@ __device__ __forceinline__ void run_tile(const MfmaArgs &a, uint8_t *As, uint32_
 				barrier_after(st);
 			}
 		} else {
-			lds_b<TYPE>(bbuf(0), bp, bi, 0, h, b);
+			lds_b<TYPE>(bbuf(0), bp, bi, k0, h, b);
 			prep(0, 0, 0);
 			for (int st = 0; st + 1 < nk; st++) {
 				steps(st, true);
 				// the last step's fragments are in registers: the barrier only
 				// waits for stage st + 1's data and this stage's LDS reads
 				barrier_after(st);
-				lds_b<TYPE>(bbuf(st + 1), bp, bi, st + 1, h, b);
+				lds_b<TYPE>(bbuf(st + 1), bp, bi, k0 + st + 1, h, b);
 				mm(L);
 				prep(st + 1, 0, L ^ 1);
 				// order: the LDS reads, two MFMAs (their latency), then the
@@ -1237,6 +1263,42 @@ __device__ __forceinline__ void run_tile(const MfmaArgs &a, uint8_t *As, uint32_
 			steps(nk - 1, false);
 			stage_barrier(); // every wave's LDS reads done before the epilogue reuses the buffers
 			mm(L);
+		}
+		if constexpr (KS > 1) {
+			// the K groups' accumulators into group 0's, in group order
+			// (16-byte words, so that a wave's accesses are contiguous)
+			typedef float f32x4 __attribute__((ext_vector_type(4)));
+			auto red = [&](int g, int mt, int j, int i) {
+				return reinterpret_cast<f32x4 *>(As0) + ((((g - 1) * NMT + mt) * 2 + j) * 4 + i) * MF_THREADS + t;
+			};
+			__syncthreads(); // every group's stage buffers free
+			if (kg > 0) {
+#pragma unroll
+				for (int mt = 0; mt < NMT; mt++)
+#pragma unroll
+					for (int j = 0; j < 2; j++)
+#pragma unroll
+						for (int i = 0; i < 4; i++)
+							*red(kg, mt, j, i) = f32x4{acc[mt][j][4 * i], acc[mt][j][4 * i + 1],
+										   acc[mt][j][4 * i + 2], acc[mt][j][4 * i + 3]};
+			}
+			__syncthreads();
+			if (kg > 0)
+				return;
+#pragma unroll
+			for (int g = 1; g < KS; g++)
+#pragma unroll
+				for (int mt = 0; mt < NMT; mt++)
+#pragma unroll
+					for (int j = 0; j < 2; j++)
+#pragma unroll
+						for (int i = 0; i < 4; i++) {
+							const f32x4 v = *red(g, mt, j, i);
+#pragma unroll
+							for (int c = 0; c < 4; c++)
+								acc[mt][j][4 * i + c] += v[c];
+						}
+			stage_barrier(); // the sums read before the epilogue's tiles overwrite them
 		}
 #ifdef TIE_MFMA_TRACE
 		bw_total = bwait;
@@ -1523,12 +1585,18 @@ __device__ __forceinline__ void run_tile(const MfmaArgs &a, uint8_t *As, uint32_
 constexpr int mf_wpe(int type, bool down, int mtr)
 {
 	return type == TIE_GGML_BF16 ? (down ? TIE_MFMA_BF16_DN_WPE : TIE_MFMA_BF16_WPE)
+	       : mtr >> 10           ? mtr >> 10
 	       : mtr == MFMA_MT_TINY ? (down ? TIE_MFMA_TINY_DN_WPC : TIE_MFMA_TINY_GU_WPC)
 	       : mtr && !down ? 3 : down ? TIE_MFMA_DN_WPE : TIE_MFMA_GU_WPE;
 }
 
+constexpr int mf_threads(int mtr)
+{
+	return MF_THREADS * (mtr >> 10 ? mtr >> 10 : 1);
+}
+
 template <int TYPE, bool DOWN, int MTR>
-__global__ __launch_bounds__(MF_THREADS) __attribute__((amdgpu_waves_per_eu(mf_wpe(TYPE, DOWN, MTR), mf_wpe(TYPE, DOWN, MTR)))) void
+__global__ __launch_bounds__(mf_threads(MTR)) __attribute__((amdgpu_waves_per_eu(mf_wpe(TYPE, DOWN, MTR), mf_wpe(TYPE, DOWN, MTR)))) void
 mfma_experts_kernel(MfmaArgs a)
 {
 	using C = Cfg<TYPE, DOWN, MTR>;
@@ -1549,7 +1617,25 @@ mfma_experts_kernel(MfmaArgs a)
 	const unsigned long long tl0 = __builtin_amdgcn_s_memrealtime();
 #endif
 	int e, slab, pbase, nrows, pair_id = 0;
-	if (MTR == MFMA_MT_TINY && a.direct) {
+	if constexpr (C::KS > 1) {
+		// a dense matrix: one expert, its pairs the dense_t tokens in order,
+		// split evenly over the tiles
+		const int nslab = gridDim.x;
+		const int ntl = (a.dense_t + a.mt_cap - 1) / a.mt_cap;
+		const int live = ntl * nslab, per_xcd = (live + 7) / 8;
+		const int lin = blockIdx.y * gridDim.x + blockIdx.x;
+		const int v = (lin % 8) * per_xcd + lin / 8;
+		if (lin / 8 >= per_xcd || v >= live)
+			return;
+		const int rpt = (a.dense_t + ntl - 1) / ntl;
+		e = 0;
+		slab = v % nslab;
+		pbase = v / nslab * rpt;
+		nrows = min(rpt, a.dense_t - pbase);
+		pair_id = pbase + (threadIdx.x % MF_THREADS);
+		if (nrows <= 0)
+			return;
+	} else if (MTR == MFMA_MT_TINY && a.direct) {
 		// one item per (expert, column slab), mapped to the workgroups in the
 		// same XCD-aware order as the tile list's items (the slabs of an
 		// expert on one XCD); the expert's count and its pair ids (at most
@@ -1991,7 +2077,7 @@ static hipError_t launch_type(const MfmaArgs &a, dim3 grid, hipStream_t s)
 			return err;
 		attr = true;
 	}
-	tie_launch((mfma_experts_kernel<TYPE, DOWN, MTR>), grid, dim3(MF_THREADS), lds, s, a);
+	tie_launch((mfma_experts_kernel<TYPE, DOWN, MTR>), grid, dim3(MF_THREADS * C::KS), lds, s, a);
 	return hipGetLastError();
 }
 
@@ -2153,18 +2239,34 @@ __global__ __launch_bounds__(RB_THREADS) void dense_prep_kernel(const float *__r
 	const float4 *xr = reinterpret_cast<const float4 *>(x + (size_t)t * in);
 	f16x8 *yr = reinterpret_cast<f16x8 *>(xa + (size_t)t * in);
 	int bad = 0;
-	for (int i = lane; i < in / 8; i += 64) {
-		const float4 a = xr[2 * i], c = xr[2 * i + 1];
-		const float m = __builtin_fmaxf(__builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(a.x), __builtin_fabsf(a.y)),
-								__builtin_fmaxf(__builtin_fabsf(a.z), __builtin_fabsf(a.w))),
-						__builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(c.x), __builtin_fabsf(c.y)),
-								__builtin_fmaxf(__builtin_fabsf(c.z), __builtin_fabsf(c.w))));
-		// fmax drops NaN: test the values themselves for NaN
-		const bool nan = a.x != a.x || a.y != a.y || a.z != a.z || a.w != a.w || c.x != c.x || c.y != c.y ||
-				 c.z != c.z || c.w != c.w;
-		bad |= (nan || !(m < 65504.0f)) ? 1 : 0;
-		yr[i] = f16x8{(_Float16)a.x, (_Float16)a.z, (_Float16)a.y, (_Float16)a.w,
-			      (_Float16)c.x, (_Float16)c.z, (_Float16)c.y, (_Float16)c.w};
+	// 4 groups of 8 values per lane requested before the first is converted
+	// (in is a multiple of 256: a group index past the row repeats the last)
+	constexpr int PG = 4;
+	for (int i0 = lane; i0 < in / 8; i0 += 64 * PG) {
+		float4 v[PG][2];
+#pragma unroll
+		for (int g = 0; g < PG; g++) {
+			const int i = min(i0 + 64 * g, in / 8 - 1);
+			v[g][0] = xr[2 * i];
+			v[g][1] = xr[2 * i + 1];
+		}
+#pragma unroll
+		for (int g = 0; g < PG; g++) {
+			const int i = i0 + 64 * g;
+			if (i >= in / 8)
+				break;
+			const float4 a = v[g][0], c = v[g][1];
+			const float m = __builtin_fmaxf(__builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(a.x), __builtin_fabsf(a.y)),
+									__builtin_fmaxf(__builtin_fabsf(a.z), __builtin_fabsf(a.w))),
+							__builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(c.x), __builtin_fabsf(c.y)),
+									__builtin_fmaxf(__builtin_fabsf(c.z), __builtin_fabsf(c.w))));
+			// fmax drops NaN: test the values themselves for NaN
+			const bool nan = a.x != a.x || a.y != a.y || a.z != a.z || a.w != a.w || c.x != c.x || c.y != c.y ||
+					 c.z != c.z || c.w != c.w;
+			bad |= (nan || !(m < 65504.0f)) ? 1 : 0;
+			yr[i] = f16x8{(_Float16)a.x, (_Float16)a.z, (_Float16)a.y, (_Float16)a.w,
+				      (_Float16)c.x, (_Float16)c.z, (_Float16)c.y, (_Float16)c.w};
+		}
 	}
 	bad = __any(bad);
 	if (lane == 0)
@@ -2210,7 +2312,28 @@ hipError_t launch_mfma_dense(const ExpertTensor &W, const float *x, int T, float
 		mt >>= 1;
 	a.mt_cap = mt;
 	const int tiles = (T + mt - 1) / mt + 1 + 8;
-	err = launch_one<true>(a, W.type, dim3(W.rows / DN_COLS, tiles), s);
+	const dim3 grid(slabs, tiles);
+	a.dense_t = T;
+	// one workgroup per CU or fewer: their 4 waves alone leave each SIMD's
+	// dequantisation, LDS reads and MFMAs in series, so the K stages go to 2
+	// or 4 groups of waves per workgroup (as many as the LDS and registers
+	// hold).  Q4_K 4096 x 2048: T=509 26.6 -> 22.5 us, T=1000 34.3 -> 29.2,
+	// T=2000 46.3 -> 41.2; Q6_K 4096 x 4096: T=500 59.1 -> 52, T=2048 96.9 ->
+	// 84.  With more workgroups than CUs two share each anyway (Q4_K 6144 x
+	// 2048, T=900: 45.5 us, split 49.4).  More stage buffers instead of the
+	// split: no gain (Q6_K 10% slower).
+	const int q4 = W.type == TIE_GGML_Q4_K;
+	if (slabs * ((T + mt - 1) / mt) > 256)
+		err = launch_one<true>(a, W.type, grid, s);
+	else if (mt == 32)
+		err = q4 ? launch_type<TIE_GGML_Q4_K, true, mfma_ks(4) | 32>(a, grid, s)
+			 : launch_type<TIE_GGML_Q6_K, true, mfma_ks(2) | 32>(a, grid, s);
+	else if (mt == 64)
+		err = q4 ? launch_type<TIE_GGML_Q4_K, true, mfma_ks(2) | 64>(a, grid, s)
+			 : launch_type<TIE_GGML_Q6_K, true, mfma_ks(2) | 64>(a, grid, s);
+	else
+		err = q4 ? launch_type<TIE_GGML_Q4_K, true, mfma_ks(2) | 128>(a, grid, s)
+			 : launch_type<TIE_GGML_Q6_K, true, mfma_ks(2) | 128>(a, grid, s);
 	if (err != hipSuccess)
 		return err;
 	return launch_dense_fix(W, x, T, out, ws.tok_flag, s);
