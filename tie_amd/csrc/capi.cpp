@@ -495,9 +495,11 @@ static bool capturing(hipStream_t s)
 }
 
 // The block on device pointers; res (optional) is added to the combine
-// (out = res + block, the residual add after the FFN).
+// (out = res + block, the residual add after the FFN); norm (optional): the
+// block runs on the RMSNorm of x.
 static int forward(tie_hip_layer *layer, const float *x, int T, int k, float *out, int32_t *idx_out,
-		   float *w_out, int flags, hipStream_t s, const float *res = nullptr, Workspace *preset = nullptr)
+		   float *w_out, int flags, hipStream_t s, const float *res = nullptr, Workspace *preset = nullptr,
+		   const NormArgs *norm = nullptr)
 {
 	if (!layer)
 		return set_error(TIE_HIP_EINVAL, "null layer");
@@ -524,6 +526,18 @@ static int forward(tie_hip_layer *layer, const float *x, int T, int k, float *ou
 	if (rc)
 		return rc;
 	Workspace &ws = *wsp;
+	// one token, one launch (eager calls on a workspace of their own: the
+	// sequence number lives on the host, so a captured graph could not
+	// advance it)
+	const bool one = !mfma && T == 1 && !preset && !capturing(s) && decode_one_supported(L, k);
+	if (norm && !(one && decode_one_norm_supported(L, k))) {
+		// (the one-launch kernel normalises its token itself)
+		prof_begin("rmsnorm", s);
+		HIP_TRY(launch_rmsnorm(x, norm->w, norm->eps, T, L.d, ws.normed, norm->tab, norm->nbits, s));
+		prof_end(s);
+		x = ws.normed;
+		norm = nullptr;
+	}
 	if (mfma) {
 		// logits (clearing the selection bytes or pair counts and the
 		// recomputation count), then selection, pair lists (small T) or
@@ -576,10 +590,7 @@ static int forward(tie_hip_layer *layer, const float *x, int T, int k, float *ou
 				HIP_TRY(launch_recompute(L, x, k, g.silu, ws.topk_idx, ws.topk_w, out, res, ws.fix_list,
 							 ws.fix_count, T, s));
 		}
-	} else if (T == 1 && !preset && !capturing(s) && decode_one_supported(L, k)) {
-		// one token, one launch (eager calls on a workspace of their own:
-		// the sequence number lives on the host, so a captured graph could
-		// not advance it)
+	} else if (one) {
 		if (++ws.one_seq == 0) {
 			HIP_TRY(hipStreamSynchronize(s));
 			HIP_TRY(hipMemset(ws.one_lg, 0, ONE_LG_COPIES * one_copy_words(ws.cap_E) * 8));
@@ -596,7 +607,7 @@ static int forward(tie_hip_layer *layer, const float *x, int T, int k, float *ou
 		}
 		HIP_TRY(launch_decode_one(L, x, k, g.silu, ws.topk_idx, ws.topk_w, out, res, ws.one_lg,
 					  one_copy_words(ws.cap_E), ws.one_h, one_copy_words((size_t)MAX_K * ws.cap_F),
-					  ws.one_seq, wseq, spin, ws.one_status, s));
+					  ws.one_seq, wseq, spin, ws.one_status, norm, s));
 	} else if (T == 1 && decode_supported(L, k)) {
 		// one token: router logits, then the experts and the combine in two
 		// launches (the selection runs in the gate/up prologue for E <= 128)
@@ -661,14 +672,12 @@ static int forward_residual(tie_hip_layer *layer, const float *hidden, const flo
 	int rc = ensure_rsqrt();
 	if (rc)
 		return rc;
-	Workspace *ws = nullptr;
-	rc = ensure_workspace(s, T, k, L.d, L.F, L.E, &ws);
-	if (rc)
-		return rc;
-	prof_begin("rmsnorm", s);
-	HIP_TRY(launch_rmsnorm(hidden, norm_w, eps, T, L.d, ws->normed, g.rsq, g.rsq_bits, s));
-	prof_end(s);
-	return forward(layer, ws->normed, T, k, out, idx_out, w_out, flags, s, hidden);
+	NormArgs norm;
+	norm.w = norm_w;
+	norm.eps = eps;
+	norm.tab = g.rsq;
+	norm.nbits = g.rsq_bits;
+	return forward(layer, hidden, T, k, out, idx_out, w_out, flags, s, hidden, nullptr, &norm);
 }
 
 } // namespace tie

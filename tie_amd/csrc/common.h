@@ -229,10 +229,21 @@ hipError_t launch_decode(const Layer &L, const float *x, int k, const float *sil
 // T = 1 in one launch (router, gate/up and down + combine workgroups that
 // hand the logits and h over as sequence-stamped words in lg / hw; E <= 128)
 bool decode_one_supported(const Layer &L, int k);
+// The RMSNorm in front of the block: its weights [d], eps and the host's
+// RSQRTSS table
+struct NormArgs {
+	const float *w = nullptr;
+	float eps = 0.0f;
+	const uint32_t *tab = nullptr;
+	int nbits = 0;
+};
+// norm (or null): x is the hidden state, normalised by the kernel itself
+// (decode_one_norm_supported)
+bool decode_one_norm_supported(const Layer &L, int k);
 hipError_t launch_decode_one(const Layer &L, const float *x, int k, const float *silu, int32_t *topk_idx,
 			     float *topk_w, float *out, const float *res, unsigned long long *lg, size_t lg_copy,
 			     unsigned long long *hw, size_t hw_copy, uint32_t seq, uint32_t wseq, int spin, int32_t *status,
-			     hipStream_t s);
+			     const NormArgs *norm, hipStream_t s);
 // polls before a wait of the one-launch decode gives up (each poll sleeps
 // about 64 cycles: tens of milliseconds in all)
 constexpr int ONE_SPIN_MAX = 1 << 18;

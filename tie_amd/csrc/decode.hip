@@ -31,6 +31,7 @@
 // padded by XPAD floats so that the segments a wave reads at once start in
 // different banks.
 #include "common.h"
+#include "rms.h"
 #include "route.h"
 
 #include <algorithm>
@@ -697,6 +698,14 @@ template <int TD> __global__ __launch_bounds__(DEC_MAX_THREADS) void decode_down
 //                    for h, then the dots and the combine (as
 //                    decode_down_kernel).
 //
+// With norm.w, x is the hidden state and the router and gate/up workgroups
+// each form its RMSNorm themselves: the router ones under their rows' loads,
+// the gate/up ones under the wait for the logits (30B: 21.0 us against 19.4
+// and 6.4 us of a launch before it; 235B, whose late gate/up workgroups find
+// the logits waiting: 52 against 44 and 9).  out may be x: a down workgroup writes its rows
+// only after every logit and every h has arrived, so after every other
+// workgroup has read x.
+//
 // Every value handed between workgroups (the E logits, the k F values of
 // h) travels as one 64-bit word {seq, value bits}, written and read with
 // agent-scope relaxed atomics (sc1: coherent across the XCDs' L2s with no
@@ -734,6 +743,7 @@ struct OneArgs {
 	uint32_t wseq;            // the stamp its waits look for (seq; another value only from the debug hook)
 	int spin;                 // polls before a wait gives up
 	int32_t *status;          // set to 1 when a wait gave up
+	NormArgs norm;            // norm.w: a.x is the hidden state, normalised in the prologues
 	int nr, ng;               // router, gate/up workgroups
 	int rpr, rg, rd;          // rows per router, gate/up, down workgroup
 };
@@ -781,6 +791,78 @@ __device__ __forceinline__ void one_select(const OneArgs &o, uint64_t *etab, int
 	topk_rank_block(o.a.E, o.a.k, etab, sel_idx, sel_w, o.a.routing, *rs, weights);
 }
 
+// The token's RMSNorm in a router workgroup: the hidden state (float4 tid +
+// i blockDim in xv[i]) to LDS row xs lane-major, the eight sum-of-squares
+// chains on lanes 0..7, then the normalised row over it.  Leaves before a
+// barrier (every thread calls it; xs is not read until the next one).
+constexpr int ONE_NX = 2;
+__device__ __forceinline__ void one_norm_lane_major(const OneArgs &o, float *xs, int n4, float4 (&xv)[ONE_NX],
+						    const float4 (&wv)[ONE_NX], float *sinv)
+{
+	const int tid = threadIdx.x, d = o.a.d, st = lane_major_stride(d);
+	auto put = [&](const float4 &v, int q) {
+		float *dst = xs + 4 * (q & 1) * st + (q >> 1);
+		dst[0] = v.x;
+		dst[st] = v.y;
+		dst[2 * st] = v.z;
+		dst[3 * st] = v.w;
+	};
+#pragma unroll
+	for (int i = 0; i < ONE_NX; i++)
+		if (tid + i * (int)blockDim.x < n4)
+			put(xv[i], tid + i * (int)blockDim.x);
+	__syncthreads();
+	if (tid < 8) {
+		const float ss = hsum8_lanes(lane_chain(xs, xs, d, tid));
+		if (tid == 0)
+			*sinv = rms_scale(ss, d, o.norm.eps, o.norm.tab, o.norm.nbits);
+	}
+	__syncthreads();
+	const float inv = *sinv;
+#pragma unroll
+	for (int i = 0; i < ONE_NX; i++)
+		if (tid + i * (int)blockDim.x < n4)
+			put(make_float4((xv[i].x * wv[i].x) * inv, (xv[i].y * wv[i].y) * inv, (xv[i].z * wv[i].z) * inv,
+					(xv[i].w * wv[i].w) * inv),
+			    tid + i * (int)blockDim.x);
+}
+
+// The same in a gate/up workgroup, on x in LDS by block ([nb][XSEG], every
+// thread's copy done before a barrier): under its wait for the logits.
+__device__ __forceinline__ void one_norm_blocks(const OneArgs &o, float *xs, float *sinv)
+{
+	const int tid = threadIdx.x, d = o.a.d, nb = d / QK;
+	__syncthreads();
+	if (tid < 8) {
+		float acc = 0.0f;
+		for (int b = 0; b < nb; b++) {
+			const float *p = xs + b * XSEG + tid;
+#pragma unroll
+			for (int i = 0; i < QK / 8; i += 16) {
+				float v[16];
+#pragma unroll
+				for (int u = 0; u < 16; u++)
+					v[u] = p[8 * (i + u)];
+#pragma unroll
+				for (int u = 0; u < 16; u++)
+					acc = __builtin_fmaf(v[u], v[u], acc);
+			}
+		}
+		const float ss = hsum8_lanes(acc);
+		if (tid == 0)
+			*sinv = rms_scale(ss, d, o.norm.eps, o.norm.tab, o.norm.nbits);
+	}
+	__syncthreads();
+	const float inv = *sinv;
+	for (int q = tid; q < d / 4; q += blockDim.x) {
+		const float4 w = reinterpret_cast<const float4 *>(o.norm.w)[q];
+		const int f = 4 * q;
+		float4 *p = reinterpret_cast<float4 *>(xs + (f / QK) * XSEG + (f % QK));
+		const float4 v = *p;
+		*p = make_float4((v.x * w.x) * inv, (v.y * w.y) * inv, (v.z * w.z) * inv, (v.w * w.w) * inv);
+	}
+}
+
 template <int TG, int TU, int TD, bool PAIR>
 __global__ __launch_bounds__(DEC_MAX_THREADS, PAIR ? ONE_PAIR_WAVES : 4) void decode_one_kernel(const OneArgs o_arg)
 {
@@ -792,6 +874,7 @@ __global__ __launch_bounds__(DEC_MAX_THREADS, PAIR ? ONE_PAIR_WAVES : 4) void de
 	__shared__ uint64_t etab[32];
 	__shared__ RankScratch rsc;
 	__shared__ int sbad;
+	__shared__ float sinv; // the RMSNorm's scale
 	const int tid = threadIdx.x, b = blockIdx.x;
 	const OneArgs &o = o_arg;
 	const DecodeArgs &a = o.a;
@@ -802,19 +885,34 @@ __global__ __launch_bounds__(DEC_MAX_THREADS, PAIR ? ONE_PAIR_WAVES : 4) void de
 		// ---- router rows e0 .. e0 + ne - 1
 		const int e0 = b * o.rpr, ne = min(o.rpr, a.E - e0);
 		const int lmf = lane_major_floats(d), st = lane_major_stride(d), n4 = d / 4;
-		// x and the rows -> LDS lane-major, all loads of a thread in flight at once
-		for (int base = tid; base < (1 + ne) * n4; base += 8 * (int)blockDim.x) {
-			float4 v[8];
+		float4 xv[ONE_NX], wv[ONE_NX];
+		if (o.norm.w) {
+			// the hidden state and the norm's weights first (n4 <= ONE_NX
+			// blockDim), so that the rows' loads below stay in flight under
+			// the sum of squares
 #pragma unroll
-			for (int i = 0; i < 8; i++) {
-				const int q = base + i * (int)blockDim.x;
+			for (int i = 0; i < ONE_NX; i++) {
+				const int c = min(tid + i * (int)blockDim.x, n4 - 1);
+				xv[i] = reinterpret_cast<const float4 *>(a.x)[c];
+				wv[i] = reinterpret_cast<const float4 *>(o.norm.w)[c];
+			}
+		}
+		// x and the rows -> LDS lane-major, all loads of a thread in flight at once
+		const int q0 = o.norm.w ? n4 : 0;
+		for (int base = q0; base < (1 + ne) * n4; base += 4 * (int)blockDim.x) {
+			float4 v[4];
+#pragma unroll
+			for (int i = 0; i < 4; i++) {
+				const int q = base + tid + i * (int)blockDim.x;
 				const int r = q / n4, c = q - r * n4;
 				const float *src = r == 0 ? a.x : o.router + (size_t)(e0 + r - 1) * d;
 				v[i] = q < (1 + ne) * n4 ? reinterpret_cast<const float4 *>(src)[c] : make_float4(0, 0, 0, 0);
 			}
+			if (o.norm.w && base == q0)
+				one_norm_lane_major(o, dl, n4, xv, wv, &sinv);
 #pragma unroll
-			for (int i = 0; i < 8; i++) {
-				const int q = base + i * (int)blockDim.x;
+			for (int i = 0; i < 4; i++) {
+				const int q = base + tid + i * (int)blockDim.x;
 				if (q < (1 + ne) * n4) {
 					const int r = q / n4, f = 4 * (q - r * n4), l = f & 7, ii = f >> 3;
 					float *dst = dl + r * lmf;
@@ -861,6 +959,8 @@ __global__ __launch_bounds__(DEC_MAX_THREADS, PAIR ? ONE_PAIR_WAVES : 4) void de
 			const int f = 4 * q;
 			*reinterpret_cast<float4 *>(xs + (f / QK) * XSEG + (f % QK)) = v;
 		});
+		if (o.norm.w)
+			one_norm_blocks(o, xs, &sinv);
 		// the experts only: their gate weights (topk_w, by the first
 		// gate/up workgroup) wait until its h is out
 		one_select(o, etab, sel_idx, sel_w, &sbad, &rsc, false);
@@ -1450,13 +1550,24 @@ int decode_one_gate_up_groups(const Layer &L, int k)
 	return (L.F / rg) * k;
 }
 
+// the kernel holds its token's hidden state in registers while it sums the
+// squares: ONE_NX float4 per thread
+bool decode_one_norm_supported(const Layer &L, int k)
+{
+	int rpr, rg, rd, threads;
+	size_t lds;
+	one_shape(L, k, one_pairs(L, k) ? 2 : 1, rpr, rg, rd, threads, lds);
+	return L.d / 4 <= ONE_NX * threads;
+}
+
 hipError_t launch_decode_one(const Layer &L, const float *x, int k, const float *silu, int32_t *topk_idx,
 			     float *topk_w, float *out, const float *res, unsigned long long *lg, size_t lg_copy,
 			     unsigned long long *hw, size_t hw_copy, uint32_t seq, uint32_t wseq, int spin, int32_t *status,
-			     hipStream_t s)
+			     const NormArgs *norm, hipStream_t s)
 {
-	OneArgs o;
-	memset(&o, 0, sizeof o);
+	OneArgs o = {};
+	if (norm)
+		o.norm = *norm;
 	DecodeArgs &a = o.a;
 	a.w[0] = L.gate.data;
 	a.w[1] = L.up.data;
