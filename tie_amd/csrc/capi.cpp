@@ -58,6 +58,8 @@ struct Ctx {
 	int32_t *idx_dev = nullptr;
 	float *norm_dev = nullptr; // [io_d] RMSNorm weights of the host-pointer residual call
 	size_t io_tokens = 0, io_d = 0, io_k = 0;
+	uint8_t *pin = nullptr; // pinned staging of the host-pointer calls of a few tokens
+	size_t pin_bytes = 0;
 	uint32_t *rsq = nullptr;   // host RSQRTSS table (built at the first residual call)
 	int rsq_bits = 0;
 	// TIE_HIP_PATH_AUTO: TIE's bit-exact kernels up to this many tokens,
@@ -251,7 +253,7 @@ static size_t carve_workspace(uint8_t *b, size_t P, size_t FF, size_t DD, size_t
 	// no-allocation entry point's scratch: that path groups h by position)
 	const size_t o_hd = direct_h ? take(EE * MFMA_DIRECT_T * FF * 2) : 0;
 	const size_t o_lg = take(ONE_LG_COPIES * one_copy_words(EE) * 8),
-		     o_dn = take(ONE_H_COPIES * one_copy_words((size_t)MAX_K * FF) * 8), o_st = take(4);
+		     o_dn = take(ONE_H_COPIES * one_copy_words((size_t)MAX_K * FF) * 8);
 	if (!b)
 		return off;
 	w->topk_idx = (int32_t *)(b + o_idx);
@@ -278,7 +280,6 @@ static size_t carve_workspace(uint8_t *b, size_t P, size_t FF, size_t DD, size_t
 	w->one_lg = (unsigned long long *)(b + o_lg);
 	w->one_h = (unsigned long long *)(b + o_dn);
 	w->one_seq = 0;
-	w->one_status = (int32_t *)(b + o_st);
 	w->cap_pairs = P;
 	w->cap_F = FF;
 	w->cap_d = DD;
@@ -300,14 +301,19 @@ static int ensure_workspace(hipStream_t s, int T, int k, int d, int F, int E, Wo
 	const size_t EE = (size_t)E > w.cap_E ? E : w.cap_E;
 	const size_t bytes = carve_workspace(nullptr, P, FF, DD, EE, nullptr);
 	void *mem = nullptr;
-	int32_t status = 0; // a given-up wait not yet reported survives the growth
+	int32_t *status = w.one_status; // (a given-up wait not yet reported survives the growth)
+	if (!status) {
+		HIP_TRY(hipHostMalloc((void **)&status, 64, hipHostMallocMapped));
+		*status = 0;
+		w.one_status = status;
+	}
 	if (w.alloc) {
 		// work still queued on s (or, through events, on any stream the
 		// caller chained to it) may read the old buffer: drain the device
 		HIP_TRY(hipDeviceSynchronize());
-		HIP_TRY(hipMemcpy(&status, w.one_status, 4, hipMemcpyDeviceToHost));
 		HIP_TRY(hipFree(w.alloc));
 		w = Workspace();
+		w.one_status = status;
 	}
 	int rc = dev_malloc(&mem, bytes, "workspace");
 	if (rc)
@@ -318,7 +324,6 @@ static int ensure_workspace(hipStream_t s, int T, int k, int d, int F, int E, Wo
 	// later one)
 	HIP_TRY(hipMemset(w.one_lg, 0, ONE_LG_COPIES * one_copy_words(EE) * 8));
 	HIP_TRY(hipMemset(w.one_h, 0, ONE_H_COPIES * one_copy_words((size_t)MAX_K * FF) * 8));
-	HIP_TRY(hipMemcpy(w.one_status, &status, 4, hipMemcpyHostToDevice));
 	return TIE_HIP_OK;
 }
 
@@ -328,15 +333,13 @@ static int ensure_workspace(hipStream_t s, int T, int k, int d, int F, int E, Wo
 static int take_stream_status(hipStream_t s)
 {
 	auto it = g.ws.find(s);
-	if (it == g.ws.end() || !it->second.alloc)
+	if (it == g.ws.end() || !it->second.one_status)
 		return TIE_HIP_OK;
 	HIP_TRY(hipStreamSynchronize(s));
-	int32_t st = 0;
-	HIP_TRY(hipMemcpy(&st, it->second.one_status, 4, hipMemcpyDeviceToHost));
-	if (!st)
+	volatile int32_t *st = it->second.one_status;
+	if (!*st)
 		return TIE_HIP_OK;
-	const int32_t zero = 0;
-	HIP_TRY(hipMemcpy(it->second.one_status, &zero, 4, hipMemcpyHostToDevice));
+	*st = 0;
 	return set_error(TIE_HIP_EHIP, "one-token forward: a wait between workgroups gave up (the GPU did not run "
 				       "them together); that call's outputs are NaN");
 }
@@ -525,7 +528,17 @@ static int forward(tie_hip_layer *layer, const float *x, int T, int k, float *ou
 	int rc = preset ? TIE_HIP_OK : ensure_workspace(s, T, k, L.d, L.F, L.E, &wsp);
 	if (rc)
 		return rc;
-	Workspace &ws = *wsp;
+	Workspace ws = *wsp;
+	// the selection straight into the caller's buffers where they allow the
+	// kernels' 16-byte accesses (else copied at the end)
+	if (idx_out && ((uintptr_t)idx_out & 15) == 0) {
+		ws.topk_idx = idx_out;
+		idx_out = nullptr;
+	}
+	if (w_out && ((uintptr_t)w_out & 15) == 0) {
+		ws.topk_w = w_out;
+		w_out = nullptr;
+	}
 	// one token, one launch (eager calls on a workspace of their own: the
 	// sequence number lives on the host, so a captured graph could not
 	// advance it)
@@ -591,13 +604,13 @@ static int forward(tie_hip_layer *layer, const float *x, int T, int k, float *ou
 							 ws.fix_count, T, s));
 		}
 	} else if (one) {
-		if (++ws.one_seq == 0) {
+		if (++wsp->one_seq == 0) {
 			HIP_TRY(hipStreamSynchronize(s));
 			HIP_TRY(hipMemset(ws.one_lg, 0, ONE_LG_COPIES * one_copy_words(ws.cap_E) * 8));
 			HIP_TRY(hipMemset(ws.one_h, 0, ONE_H_COPIES * one_copy_words((size_t)MAX_K * ws.cap_F) * 8));
-			ws.one_seq = 1;
+			wsp->one_seq = 1;
 		}
-		uint32_t wseq = ws.one_seq;
+		uint32_t wseq = wsp->one_seq;
 		int spin = ONE_SPIN_MAX;
 		if (g.debug_stale > 0) {
 			// debug hook: wait for a stamp no workgroup writes, briefly
@@ -607,7 +620,7 @@ static int forward(tie_hip_layer *layer, const float *x, int T, int k, float *ou
 		}
 		HIP_TRY(launch_decode_one(L, x, k, g.silu, ws.topk_idx, ws.topk_w, out, res, ws.one_lg,
 					  one_copy_words(ws.cap_E), ws.one_h, one_copy_words((size_t)MAX_K * ws.cap_F),
-					  ws.one_seq, wseq, spin, ws.one_status, norm, s));
+					  wsp->one_seq, wseq, spin, ws.one_status, norm, s));
 	} else if (T == 1 && decode_supported(L, k)) {
 		// one token: router logits, then the experts and the combine in two
 		// launches (the selection runs in the gate/up prologue for E <= 128)
@@ -726,10 +739,17 @@ extern "C" void tie_hip_shutdown(void)
 	for (auto &kv : g.cache)
 		free_layer(kv.second);
 	g.cache.clear();
-	for (auto &kv : g.ws)
+	for (auto &kv : g.ws) {
 		if (kv.second.alloc)
 			(void)hipFree(kv.second.alloc);
+		if (kv.second.one_status)
+			(void)hipHostFree(kv.second.one_status);
+	}
 	g.ws.clear();
+	if (g.pin)
+		(void)hipHostFree(g.pin);
+	g.pin = nullptr;
+	g.pin_bytes = 0;
 	for (void *p : {(void *)g.x_dev, (void *)g.out_dev, (void *)g.w_dev, (void *)g.idx_dev, (void *)g.silu,
 			(void *)g.norm_dev, (void *)g.rsq})
 		if (p)
@@ -828,6 +848,10 @@ extern "C" int tie_hip_moe_forward_noalloc(tie_hip_layer *layer, const float *x_
 	return forward(layer, x_dev, T, k, out_dev, topk_idx_dev, topk_w_dev, flags, s, nullptr, &ws);
 }
 
+// x of the host-buffer calls that go through pinned staging, at most (above,
+// the copies' bandwidth counts, not their latency)
+constexpr size_t PIN_MAX = (size_t)256 << 10;
+
 // The host-buffer drop-ins: the layer comes from the weight cache (uploaded
 // at the first call with these weights), x goes up, out and the selection
 // come back, and the call returns after the stream has drained.
@@ -900,6 +924,63 @@ static int moe_ffn_host(const float *x, int T, int d, int F, int E, int k, const
 		g.io_tokens = nt;
 		g.io_d = nd;
 		g.io_k = nk;
+	}
+	const size_t nx = (size_t)T * d * 4, nk = (size_t)T * k * 4, nn = ffn_norm ? (size_t)d * 4 : 0;
+	if (nx <= PIN_MAX) {
+		// a few tokens: through pinned memory that the kernels read and write
+		// themselves (copies from and to pageable memory each hold the host
+		// until they are done: 30B T=1 with norm and selection 120 us a call,
+		// of which the kernels 28)
+		const size_t ax = align256(nx), an = align256(nn), ak = align256(nk), need = 2 * ax + an + 2 * ak;
+		if (need > g.pin_bytes) {
+			if (g.pin)
+				HIP_TRY(hipHostFree(g.pin)); // (every call leaves the stream drained)
+			g.pin = nullptr;
+			g.pin_bytes = 0;
+			HIP_TRY(hipHostMalloc((void **)&g.pin, need, hipHostMallocMapped));
+			g.pin_bytes = need;
+		}
+		uint8_t *hx = g.pin, *hn = hx + ax, *ho = hn + an, *hi = ho + ax, *hw = hi + ak;
+		memcpy(hx, x, nx);
+		if (nn)
+			memcpy(hn, ffn_norm, nn);
+		CopyRuns in;
+		in.src[0] = hx;
+		in.dst[0] = g.x_dev;
+		in.n[0] = (int)(nx / 4);
+		in.src[1] = hn;
+		in.dst[1] = g.norm_dev;
+		in.n[1] = (int)(nn / 4);
+		HIP_TRY(launch_copy_runs(in, g.stream));
+		// the one-launch decode only writes the selection; the kernels of more
+		// tokens read it back, so theirs stays on the device until the end
+		const bool direct = T == 1 && decode_one_supported(layer->L, k) && g.exact_max_t >= 1;
+		int32_t *oi = !topk_idx_opt ? nullptr : direct ? (int32_t *)hi : g.idx_dev;
+		float *ow = !topk_w_opt ? nullptr : direct ? (float *)hw : g.w_dev;
+		rc = ffn_norm ? forward_residual(layer, g.x_dev, g.norm_dev, eps, T, k, (float *)ho, oi, ow, TIE_HIP_PATH_AUTO,
+						 g.stream)
+			      : forward(layer, g.x_dev, T, k, (float *)ho, oi, ow, TIE_HIP_PATH_AUTO, g.stream);
+		if (rc == TIE_HIP_OK && !direct && (oi || ow)) {
+			CopyRuns sel;
+			sel.src[0] = oi;
+			sel.dst[0] = hi;
+			sel.n[0] = oi ? T * k : 0;
+			sel.src[1] = ow;
+			sel.dst[1] = hw;
+			sel.n[1] = ow ? T * k : 0;
+			HIP_TRY(launch_copy_runs(sel, g.stream));
+		}
+		// (drained on an error too: the staging may be freed by the next call)
+		const hipError_t e = hipStreamSynchronize(g.stream);
+		if (rc)
+			return rc;
+		HIP_TRY(e);
+		memcpy(out, ho, nx);
+		if (topk_idx_opt)
+			memcpy(topk_idx_opt, hi, nk);
+		if (topk_w_opt)
+			memcpy(topk_w_opt, hw, nk);
+		return take_stream_status(g.stream);
 	}
 	HIP_TRY(hipMemcpyAsync(g.x_dev, x, (size_t)T * d * 4, hipMemcpyHostToDevice, g.stream));
 	if (ffn_norm) {
@@ -1232,6 +1313,9 @@ extern "C" int tie_hip_stream_release(void *stream)
 	HIP_TRY(hipDeviceSynchronize());
 	if (it->second.alloc)
 		HIP_TRY(hipFree(it->second.alloc));
+	it->second.alloc = nullptr;
+	if (it->second.one_status)
+		HIP_TRY(hipHostFree(it->second.one_status));
 	g.ws.erase(it);
 	return TIE_HIP_OK;
 }

@@ -131,7 +131,9 @@ struct Workspace {
 	unsigned long long *one_lg = nullptr; // [ONE_LG_COPIES][E, 4 KiB rows]  one-launch decode: {seq, logit} words
 	unsigned long long *one_h = nullptr; // [ONE_H_COPIES][MAX_K * F, 4 KiB rows] one-launch decode: {seq, h} words
 	uint32_t one_seq = 0;         // one-launch decode: sequence number of the last call
-	int32_t *one_status = nullptr; // [1] one-launch decode: 1 when a wait gave up (outputs NaN)
+	int32_t *one_status = nullptr; // [1] one-launch decode: 1 when a wait gave up (outputs NaN); pinned host
+	                               //     memory, kept when the workspace grows (the no-allocation scratch, where
+	                               //     that kernel does not run, has none)
 	size_t cap_pairs = 0, cap_F = 0, cap_d = 0, cap_E = 0;
 	void *alloc = nullptr;
 };
@@ -288,6 +290,15 @@ int dense_groups(int T);
 hipError_t launch_combine(int T, int d, int k, const float *topk_w, const int32_t *topk_idx, const float *y,
 			  float *out, hipStream_t s, const float *res = nullptr, const int32_t *skip = nullptr,
 			  bool y16 = false, int y_shift = 0);
+// dst[i] = src[i] for up to three runs of 4-byte words, by one small kernel
+// (16-byte accesses where a run's pointers allow them): pinned host memory to
+// and from the device without the latency of a copy engine's commands
+struct CopyRuns {
+	const void *src[3] = {};
+	void *dst[3] = {};
+	int n[3] = {}; // words
+};
+hipError_t launch_copy_runs(const CopyRuns &r, hipStream_t s);
 // TIE's RMSNorm of each row of x into out; tab/nbits: the host RSQRTSS table
 hipError_t launch_rmsnorm(const float *x, const float *w, float eps, int T, int d, float *out, const uint32_t *tab,
 			  int nbits, hipStream_t s);

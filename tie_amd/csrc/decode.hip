@@ -712,7 +712,7 @@ template <int TD> __global__ __launch_bounds__(DEC_MAX_THREADS) void decode_down
 // cache write-back, invalidate or separate flag); seq (one per call) tells
 // a word of this call from one left by an earlier call.  The waits are
 // bounded (spin polls): a wait that gives up produces NaN outputs instead
-// of hanging, and sets the call's status word, which the host reads back
+// of hanging, and sets the call's status word in pinned host memory
 // (tie_hip_stream_status; the synchronous entry points return the error).
 
 __device__ __forceinline__ unsigned long long ld_word(const unsigned long long *p)
@@ -1001,7 +1001,7 @@ __global__ __launch_bounds__(DEC_MAX_THREADS, PAIR ? ONE_PAIR_WAVES : 4) void de
 						   __HIP_MEMORY_SCOPE_AGENT);
 		}
 		if (sbad && tid == 0)
-			__hip_atomic_store(o.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+			__hip_atomic_store(o.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 		if (gb == 0) {
 			topk_rank_weights(a.k, etab, sel_idx, sel_w, a.routing, rsc);
 			if (tid < a.k) {
@@ -1102,7 +1102,7 @@ __global__ __launch_bounds__(DEC_MAX_THREADS, PAIR ? ONE_PAIR_WAVES : 4) void de
 	if (sbad && tid < R)
 		outp[tid] = __builtin_nanf("");
 	if (sbad && tid == 0)
-		__hip_atomic_store(o.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		__hip_atomic_store(o.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 #ifdef TIE_ONE_TRACE
 	if (tid == 0) {
 		ONE_T(t_end);

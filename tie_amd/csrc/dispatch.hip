@@ -14,6 +14,8 @@
 // The combine then restores token order: out[t] = sum_j g[t][j] * y[t*k+j]
 // in slot order j = 0..k-1 with one FMA per term, as model_qwen3.c:459-467
 // does (acc starts at +0.0f; slots with no expert contribute nothing).
+#include <algorithm>
+
 #include "common.h"
 #include "route.h"
 
@@ -246,6 +248,38 @@ hipError_t launch_combine(int T, int d, int k, const float *topk_w, const int32_
 	const int n4 = d / 4;
 	tie_launch(combine_kernel, dim3((n4 + 255) / 256, T), dim3(256), 0, s, T, d, k, topk_w, topk_idx, y, res,
 			   out, skip);
+	return hipGetLastError();
+}
+
+// ------------------------------------------------------------ copy_runs
+// Bound by the host link's latency at the sizes it serves (x of a few tokens:
+// 8 KiB to 256 KiB): about 4 us with its launch, where two asynchronous
+// copies from pageable memory held the host for 20 us and more.
+constexpr int CP_THREADS = 256;
+__global__ __launch_bounds__(CP_THREADS) void copy_runs_kernel(const CopyRuns r)
+{
+	const int i0 = blockIdx.x * CP_THREADS + threadIdx.x, step = gridDim.x * CP_THREADS;
+#pragma unroll
+	for (int k = 0; k < 3; k++) {
+		const int n = r.n[k];
+		const uint32_t *s = reinterpret_cast<const uint32_t *>(r.src[k]);
+		uint32_t *d = reinterpret_cast<uint32_t *>(r.dst[k]);
+		const bool wide = (((uintptr_t)s | (uintptr_t)d) & 15) == 0;
+		const int n4 = wide ? n / 4 : 0;
+		for (int i = i0; i < n4; i += step)
+			reinterpret_cast<uint4 *>(d)[i] = reinterpret_cast<const uint4 *>(s)[i];
+		for (int i = 4 * n4 + i0; i < n; i += step)
+			d[i] = s[i];
+	}
+}
+
+hipError_t launch_copy_runs(const CopyRuns &r, hipStream_t s)
+{
+	const int most = std::max(r.n[0], std::max(r.n[1], r.n[2]));
+	if (most == 0)
+		return hipSuccess;
+	const int wg = std::min(256, std::max(1, most / (4 * CP_THREADS)));
+	tie_launch(copy_runs_kernel, dim3(wg), dim3(CP_THREADS), 0, s, r);
 	return hipGetLastError();
 }
 
