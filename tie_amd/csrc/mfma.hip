@@ -299,6 +299,17 @@ template <int TYPE, bool DOWN = false, int MTR = 0> struct Cfg {
 				  : 4 * (ABUF + BBUF) + ROFF_BYTES <= LDS_BUDGET ? 4
 				  : 3 * (ABUF + BBUF) + ROFF_BYTES <= LDS_BUDGET ? 3 : 2;
 	static_assert(NWAVES == 4, "epilogue tile size");
+	// A block's scales (and Q6_K's d and, per half, qh) are moved and read
+	// into registers once, in the first stage that needs them, and stay there
+	// for the block's other stages (two stage buffers: no barrier counts the
+	// loads in flight); the stage loops are unrolled by the block, so the
+	// sub-block arithmetic of the scales is constant too.  Read again in every
+	// stage, these chunks were a third of Q6_K's L2-to-LDS bytes and a quarter
+	// of Q4_K's.  Kernels, one box, without / with: down (Q6_K) 30B T=32 34.9 /
+	// 32.8 us, T=101 41.4 / 39.0, T=500 52.8 / 47.5, T=2048 104.7 / 97.0, 235B
+	// T=1024 208 / 190; gate/up (Q4_K) T=32 43.8 / 42.2, T=256 56.2 / 51.7,
+	// T=2048 147.7 / 146.4, 235B T=1024 304 / 292; Q4_K down T=500 41.5 / 39.3
+	static constexpr bool RES = F16 && KST == 64 && KS == 1 && NS == 2 && QK / KST == 4;
 	// DMA instructions one wave issues per weight stage (dma_b)
 	static constexpr int B_DMA = NCH + (TYPE == TIE_GGML_Q6_K ? 1 : 0);
 	static constexpr int LDS_A = NS * ABUF, LDS_B = B_LDS ? NS * BBUF : 0;
@@ -338,7 +349,7 @@ template <> struct BRegs<TIE_GGML_Q4_K> {
 template <> struct BRegs<TIE_GGML_Q6_K> {
 	u32x4 ql[2][2]; // ql chunks 2c + h of the stage's ql slots, c < ql slots / 2
 	u32x4 qh[2];    // qh chunk h of the half
-	u32x2 sc[2];    // the half's 8 scales
+	u32x4 sc[2];    // the 16 scales, or (not block-resident) the half's 8 in .xy
 	uint32_t d[2];  // fp16 d
 };
 template <> struct BRegs<TIE_GGML_BF16> {
@@ -369,105 +380,110 @@ __device__ __forceinline__ void load_b(const BSrc &s, int st, int h, BRegs<TYPE>
 // The stage's weight chunks of the workgroup's 4 panels -> LDS buffer B:
 // panel p (gate/up: gate panels 0, 1 and up panels 2, 3 of the tile's 128
 // columns; down: 4 panels of its 256 columns), chunk slot c, 1 KiB each.
-// Q4_K slots: 0 scales, 1..4 the stage's quant chunks 1+4h..4+4h.  Q6_K
-// slots: 0..3 ql chunks 4h..4h+3, 4, 5 qh chunks 8+2h, 9+2h, 6 the scales;
-// then the 4 panels' d planes (128 B each).  h = st % 2 (the block half).
-// Wave w moves items 4c + w (panel (4c + w) / NCH, slot (4c + w) % NCH);
-// their bases and panel offsets are set once per tile (BDma).
-template <int TYPE, int MTR = 0> struct BDma {
-	static constexpr int NCH = Cfg<TYPE, false, MTR>::NCH;
-	const uint8_t *base[NCH]; // expert base of the item's matrix (wave-uniform)
-	uint32_t pofs[NCH];       // the item's panel row offset in the expert (wave-uniform)
-	int slot[NCH];            // the item's LDS slot
-	uint32_t lofs[NCH];       // the item's LDS offset in a B buffer
-	uint32_t lane16;          // 16 * lane
-	const uint8_t *dbase;     // Q6_K: expert base of panel w's matrix
-	uint32_t dpofs;           // Q6_K: offset of panel w's d plane in its first block column
+// Q4_K slots: 0 scales, 1, 2 the stage's quant chunks.  Q6_K slots: 0, 1 the
+// stage's ql chunks, 2, 3 the block half's qh chunks, 4 the scales; then the 4
+// panels' d planes (128 B each).  Parts that a block's later stages use too
+// are moved once (Cfg::RES).
+// Wave w moves panel w's chunks; their base and panel offset are set once per
+// tile (BDma).
+struct BDma {
+	const uint8_t *base; // expert base of panel w's matrix (wave-uniform)
+	uint32_t pofs;       // the panel row's offset in the expert (wave-uniform)
+	uint32_t lane16;     // 16 * lane
 };
 
-template <int TYPE, bool DOWN, int MTR = 0>
-__device__ __forceinline__ void bdma_init(const MfmaArgs &a, int e, int slab, int w, BDma<TYPE, MTR> &d)
+template <int TYPE, bool DOWN>
+__device__ __forceinline__ void bdma_init(const MfmaArgs &a, int e, int slab, int w, BDma &d)
 {
-	using C = Cfg<TYPE, false, MTR>;
-	const uint32_t pbytes = (uint32_t)panel_bytes(TYPE);
-	const uint32_t nkb = (uint32_t)(a.in / QK);
-#pragma unroll
-	for (int c = 0; c < C::NCH; c++) {
-		const int it = NWAVES * c + w; // NWAVES == 4 panels
-		const int p = it / C::NCH, s = it % C::NCH;
-		const int mat = DOWN ? 0 : p >> 1;
-		const int rt = DOWN ? 4 * slab + p : 2 * slab + (p & 1);
-		d.base[c] = a.w[mat] + (size_t)e * a.expert_bytes[mat];
-		d.pofs[c] = (uint32_t)rt * nkb * pbytes;
-		d.slot[c] = s;
-		d.lofs[c] = (uint32_t)(p * C::PB + s * 1024);
-	}
+	const int mat = DOWN ? 0 : w >> 1;
+	const int rt = DOWN ? 4 * slab + w : 2 * slab + (w & 1);
+	d.base = a.w[mat] + (size_t)e * a.expert_bytes[mat];
+	d.pofs = (uint32_t)rt * (uint32_t)(a.in / QK) * (uint32_t)panel_bytes(TYPE);
 	d.lane16 = 16u * (threadIdx.x & 63);
-	{
-		const int mat = DOWN ? 0 : w >> 1;
-		const int rt = DOWN ? 4 * slab + w : 2 * slab + (w & 1);
-		d.dbase = a.w[mat] + (size_t)e * a.expert_bytes[mat];
-		d.dpofs = (uint32_t)rt * nkb * pbytes + Q6K_CHUNKS * 1024;
-	}
+}
+
+// Whether stage st (mod the stages per block) reads slot c of a panel from
+// LDS (C::RES: block-resident parts only in the first stage that needs them);
+// c = -1: the Q6_K d plane
+template <int TYPE, typename C> __device__ constexpr bool slot_moved(int st, int c)
+{
+	if (!C::RES)
+		return true;
+	if (TYPE == TIE_GGML_Q4_K)
+		return c != 0 || st % C::SPB == 0;
+	return c < 0 || c == 4 ? st % C::SPB == 0 : c < 2 || (st & 1) == 0;
 }
 
 template <int TYPE, bool DOWN, int MTR = 0>
-__device__ __forceinline__ void dma_b(const BDma<TYPE, MTR> &d, int slab, int st, int w, uint8_t *B)
+__device__ __forceinline__ void dma_b(const BDma &d, int st, int sb, int w, uint8_t *B)
 {
-	using C = Cfg<TYPE, false, MTR>;
-	const int half = st & 1, part = st % C::SPB;
+	using C = Cfg<TYPE, DOWN, MTR>;
+	const int half = sb & 1, part = sb % C::SPB;
 	const uint32_t kofs = (uint32_t)(st / C::SPB) * (uint32_t)panel_bytes(TYPE);
-	const uint32_t lb = lds_addr(B);
+	const uint32_t lb = lds_addr(B) + w * C::PB;
 #pragma unroll
-	for (int c = 0; c < C::NCH; c++) {
-		const int s = d.slot[c];
+	for (int s = 0; s < C::NCH; s++) {
+		if (!slot_moved<TYPE, C>(sb, s))
+			continue;
 		int chunk;
 		if constexpr (TYPE == TIE_GGML_Q4_K)
 			chunk = s == 0 ? 0 : (C::NCH - 1) * part + s;
 		else if constexpr (C::APERM) {
 			// ql chunks of quarters q, q + 2 of half n; the half's qh; scales
-			const int n = (st >> 1) & 1, q = st & 1;
+			const int n = (sb >> 1) & 1, q = sb & 1;
 			chunk = s < 2 ? 4 * n + 2 * q + s : (s < 4 ? 8 + 2 * n + (s - 2) : 12);
 		} else
 			chunk = s < 4 ? 4 * half + s : (s < 6 ? 8 + 2 * half + (s - 4) : 12);
-		dma16s(d.base[c], d.lane16 + (d.pofs[c] + kofs + (uint32_t)chunk * 1024),
-		       __builtin_amdgcn_readfirstlane(lb + d.lofs[c]));
+		dma16s(d.base, d.lane16 + (d.pofs + kofs + (uint32_t)chunk * 1024),
+		       __builtin_amdgcn_readfirstlane(lb + s * 1024));
 	}
 	if constexpr (TYPE == TIE_GGML_Q6_K) {
 		// the d plane of panel w (128 B)
-		if ((threadIdx.x & 63) < 8)
-			dma16s(d.dbase, d.lane16 + (d.dpofs + kofs), __builtin_amdgcn_readfirstlane(lb + 4 * C::PB + w * 128));
+		if (slot_moved<TYPE, C>(sb, -1) && (threadIdx.x & 63) < 8)
+			dma16s(d.base, d.lane16 + (d.pofs + kofs + Q6K_CHUNKS * 1024),
+			       __builtin_amdgcn_readfirstlane(lds_addr(B) + 4 * C::PB + w * 128));
 	}
 }
 
 // The lane's weights of the stage from LDS buffer B: row j of the lane in
 // panel p[j], slot i[j].
-template <int TYPE, int MTR = 0>
+template <int TYPE, bool DOWN, int MTR>
 __device__ __forceinline__ void lds_b(const uint8_t *B, const int p[2], const int i[2], int st, int h, BRegs<TYPE> &b)
 {
-	using C = Cfg<TYPE, false, MTR>;
+	using C = Cfg<TYPE, DOWN, MTR>;
 #pragma unroll
 	for (int j = 0; j < 2; j++) {
 		const uint8_t *pb = B + p[j] * C::PB + i[j] * 16;
-		if constexpr (TYPE == TIE_GGML_Q4_K && C::UH) {
-			// both code chunks of the stage's group (the lane half takes its nibble)
-			b.q[j][0] = *reinterpret_cast<const u32x4 *>(pb + 1024);
-			b.q[j][1] = *reinterpret_cast<const u32x4 *>(pb + 2 * 1024);
-			b.sc[j] = *reinterpret_cast<const u32x4 *>(pb);
-		} else if constexpr (TYPE == TIE_GGML_Q4_K) {
+		if constexpr (TYPE == TIE_GGML_Q4_K) {
+			if constexpr (C::UH) {
+				// both code chunks of the stage's group (the lane half takes its nibble)
+				b.q[j][0] = *reinterpret_cast<const u32x4 *>(pb + 1024);
+				b.q[j][1] = *reinterpret_cast<const u32x4 *>(pb + 2 * 1024);
+			} else {
 #pragma unroll
-			for (int g = 0; g < (C::NCH - 1) / 2; g++)
-				b.q[j][g] = *reinterpret_cast<const u32x4 *>(pb + (1 + 2 * g + h) * 1024);
-			b.sc[j] = *reinterpret_cast<const u32x4 *>(pb);
+				for (int g = 0; g < (C::NCH - 1) / 2; g++)
+					b.q[j][g] = *reinterpret_cast<const u32x4 *>(pb + (1 + 2 * g + h) * 1024);
+			}
+			if (slot_moved<TYPE, C>(st, 0))
+				b.sc[j] = *reinterpret_cast<const u32x4 *>(pb);
 		} else if constexpr (TYPE == TIE_GGML_Q6_K) {
 			constexpr int NQL = C::APERM ? 2 : 4; // ql chunk slots
 #pragma unroll
 			for (int c = 0; c < NQL / 2; c++)
 				b.ql[j][c] = *reinterpret_cast<const u32x4 *>(pb + (2 * c + h) * 1024);
-			b.qh[j] = *reinterpret_cast<const u32x4 *>(pb + (NQL + h) * 1024);
-			const int half = C::APERM ? (st >> 1) & 1 : st & 1;
-			b.sc[j] = *reinterpret_cast<const u32x2 *>(pb + (NQL + 2) * 1024 + 8 * half);
-			b.d[j] = *reinterpret_cast<const uint16_t *>(B + 4 * C::PB + p[j] * 128 + 2 * i[j]);
+			if (slot_moved<TYPE, C>(st, 2))
+				b.qh[j] = *reinterpret_cast<const u32x4 *>(pb + (NQL + h) * 1024);
+			if (slot_moved<TYPE, C>(st, 4)) {
+				if constexpr (C::RES)
+					b.sc[j] = *reinterpret_cast<const u32x4 *>(pb + (NQL + 2) * 1024);
+				else {
+					const int half = C::APERM ? (st >> 1) & 1 : st & 1;
+					const u32x2 sc = *reinterpret_cast<const u32x2 *>(pb + (NQL + 2) * 1024 + 8 * half);
+					b.sc[j].x = sc.x;
+					b.sc[j].y = sc.y;
+				}
+				b.d[j] = *reinterpret_cast<const uint16_t *>(B + 4 * C::PB + p[j] * 128 + 2 * i[j]);
+			}
 		}
 	}
 }
@@ -726,7 +742,7 @@ __device__ __forceinline__ void deq_step(const BRegs<TYPE> &b, const Fac &f, int
 // lo, hi, as in deq_step) -> f16 pairs (K 0,2), (1,3), (4,6), (5,7): a code
 // in the mantissa of 1024.0, minus 1056 = code - 32 (exact), times
 // d * sc * 2^F16_SHIFT (v_pk_mul_f16, one rounding).
-template <bool NOD = false> // NOD: without the factor d 2^S ((q - 32) sc, exact)
+template <bool NOD, bool RES> // NOD: without the factor d 2^S ((q - 32) sc, exact)
 __device__ __forceinline__ void deq_step16_q6k(const BRegs<TIE_GGML_Q6_K> &b, const Fac &f, const K16 &kc, int st, int s,
 					       f16x8 out[2])
 {
@@ -746,7 +762,9 @@ __device__ __forceinline__ void deq_step16_q6k(const BRegs<TIE_GGML_Q6_K> &b, co
 		const uint32_t lo = ((ql.x >> nsh) & 0x0f0f0f0fu) | (qhs(qh.x) & 0xf0f0f0f0u);
 		const uint32_t hi = ((ql.y >> nsh) & 0x0f0f0f0fu) | (qhs(qh.y) & 0xf0f0f0f0u);
 		// scale 2r + h: positions 16 h + 8 (s % 2) + i of the quarter
-		const uint32_t sw = r < 2 ? b.sc[j].x : b.sc[j].y;
+		// (block-resident scales: all 16, the half a constant)
+		const int hs = RES ? (st >> 1) & 1 : 0;
+		const uint32_t sw = hs ? (r < 2 ? b.sc[j].z : b.sc[j].w) : (r < 2 ? b.sc[j].x : b.sc[j].y);
 		// (q - 32) sc exact in f16 (|sc| <= 64: |(q - 32) sc| <= 2048), then
 		// times d 2^S with one rounding: d sc is not rounded to f16 first
 		const f16x2 SC = splat16((float)(int8_t)((sw >> (16 * (r & 1) + 8 * lane_half())) & 0xffu));
@@ -938,7 +956,7 @@ template <int TYPE, bool DOWN, int MTR> struct Ops<TYPE, DOWN, MTR, true> {
 		if constexpr (TYPE == TIE_GGML_Q4_K)
 			deq_step16<Cfg<TYPE, DOWN, MTR>::UH, NOD>(b, f, kc, s, out);
 		else
-			deq_step16_q6k<NOD>(b, f, kc, st, s, out);
+			deq_step16_q6k<NOD, Cfg<TYPE, DOWN, MTR>::RES>(b, f, kc, st, s, out);
 	}
 	__device__ static f32x16 mma(V a, V b, f32x16 c)
 	{
@@ -1088,16 +1106,18 @@ __device__ __forceinline__ void run_tile(const MfmaArgs &a, uint8_t *As, uint32_
 		using V = typename O::V;
 		constexpr int NA = NMT;
 		static_assert(C::NPL == 1 && C::NSTEP % 2 == 0, "one activation plane, even step count");
-		BDma<TYPE, MTR> bd;
-		bdma_init<TYPE, DOWN, MTR>(a, e, slab, w, bd);
+		BDma bd;
+		bdma_init<TYPE, DOWN>(a, e, slab, w, bd);
 		constexpr int NS = C::NS;
 		auto abuf = [&](int st) { return As + (st % NS) * C::ABUF; };
 		auto bbuf = [&](int st) { return Bs + (st % NS) * C::BBUF; };
 		// stage st's activations and weights into buffers st % NS
-		auto issue = [&](int st) {
+		// (sb: st mod the stages per block, or st + k0; a constant where the
+		// stage loop is unrolled by the block)
+		auto issue = [&](int st, int sb) {
 			if (st < nk) {
 				dma_a<TYPE, DOWN, NMT, MTR>(as, k0 + st, w, abuf(st));
-				dma_b<TYPE, DOWN, MTR>(bd, slab, k0 + st, w, bbuf(st));
+				dma_b<TYPE, DOWN, MTR>(bd, k0 + st, sb, w, bbuf(st));
 			}
 		};
 		// direct loads one wave issues per stage (dma_a + dma_b)
@@ -1135,11 +1155,11 @@ __device__ __forceinline__ void run_tile(const MfmaArgs &a, uint8_t *As, uint32_
 		// with the minimum term from the sub-block sums)
 		constexpr bool DF = TIE_MFMA_DFOLD && TYPE == TIE_GGML_Q6_K && NMT == 1 && MTR == MFMA_MT_TINY;
 		constexpr bool QF = TIE_MFMA_QFOLD && C::UH && !DOWN && NMT == 1 && MTR == MFMA_MT_TINY;
-		auto prep = [&](int st, int s, int slot) {
+		auto prep = [&](int st, int sb, int s, int slot) {
 			read(st, s, fa[slot]);
 			if (s == 0 || (TYPE == TIE_GGML_Q4_K && s % 4 == 0))
-				O::factors(b, k0 + st, s / 4, f);
-			O::template deq<DF || QF>(b, f, kc, k0 + st, s, fb[slot]);
+				O::factors(b, sb, s / 4, f);
+			O::template deq<DF || QF>(b, f, kc, sb, s, fb[slot]);
 		};
 		auto mm = [&](int slot) {
 #pragma unroll
@@ -1151,21 +1171,21 @@ __device__ __forceinline__ void run_tile(const MfmaArgs &a, uint8_t *As, uint32_
 		constexpr int L = (C::NSTEP - 1) & 1; // slot of a stage's last step
 		// all steps but the last of stage st (the DMA of stage st + NS - 1
 		// with more)
-		auto steps = [&](int st, bool more) {
+		auto steps = [&](int st, int sb, bool more) {
 #pragma unroll
 			for (int s = 0; s + 1 < C::NSTEP; s++) {
 				mm(s & 1);
 				// the buffers written here were last read in stage st - 1,
 				// which every wave has left (its barrier)
 				if (s == 0 && more)
-					issue(st + NS - 1);
-				prep(st, s + 1, (s & 1) ^ 1);
+					issue(st + NS - 1, sb + NS - 1);
+				prep(st, sb, s + 1, (s & 1) ^ 1);
 				__builtin_amdgcn_sched_barrier(0);
 			}
 		};
 #pragma unroll
 		for (int i = 0; i + 1 < NS; i++)
-			issue(i);
+			issue(i, k0 + i);
 		barrier_after(-1);
 		if constexpr (DF || QF) {
 			// as below, block by block: the block's MFMAs into accb (from
@@ -1187,9 +1207,9 @@ __device__ __forceinline__ void run_tile(const MfmaArgs &a, uint8_t *As, uint32_
 #pragma unroll
 				for (int sb = 0; sb < C::SPB; sb++) {
 					const int st = st0 + sb;
-					issue(st + NS - 1);
-					lds_b<TYPE, MTR>(bbuf(st), bp, bi, k0 + st, h, b);
-					prep(st, 0, 0);
+					issue(st + NS - 1, sb + NS - 1);
+					lds_b<TYPE, DOWN, MTR>(bbuf(st), bp, bi, sb, h, b);
+					prep(st, sb, 0, 0);
 #pragma unroll
 					for (int s = 0; s < C::NSTEP; s++) {
 #pragma unroll
@@ -1197,7 +1217,7 @@ __device__ __forceinline__ void run_tile(const MfmaArgs &a, uint8_t *As, uint32_
 							accb[j] = O::mma(fa[s & 1][0], fb[s & 1][j],
 									 (sb == 0 && s == 0) ? f32x16{} : accb[j]);
 						if (s + 1 < C::NSTEP)
-							prep(st, s + 1, (s & 1) ^ 1);
+							prep(st, sb, s + 1, (s & 1) ^ 1);
 						__builtin_amdgcn_sched_barrier(0);
 					}
 					if (sb + 1 == C::SPB) {
@@ -1225,30 +1245,39 @@ __device__ __forceinline__ void run_tile(const MfmaArgs &a, uint8_t *As, uint32_
 		} else if constexpr (NMT < TIE_MFMA_PIPE_NMT) {
 			// few MFMAs per step: each stage self-contained (the DMA of stage
 			// st + NS - 1 first, then its weights from LDS, then the steps)
-			for (int st = 0; st < nk; st++) {
-				issue(st + NS - 1);
-				lds_b<TYPE, MTR>(bbuf(st), bp, bi, k0 + st, h, b);
-				prep(st, 0, 0);
+			auto stage = [&](int st, int sb) {
+				issue(st + NS - 1, sb + NS - 1);
+				lds_b<TYPE, DOWN, MTR>(bbuf(st), bp, bi, sb, h, b);
+				prep(st, sb, 0, 0);
 #pragma unroll
 				for (int s = 0; s < C::NSTEP; s++) {
 					mm(s & 1);
 					if (s + 1 < C::NSTEP)
-						prep(st, s + 1, (s & 1) ^ 1);
+						prep(st, sb, s + 1, (s & 1) ^ 1);
 					__builtin_amdgcn_sched_barrier(0);
 				}
 				barrier_after(st);
+			};
+			if constexpr (C::RES) {
+				for (int st0 = 0; st0 < nk; st0 += C::SPB)
+#pragma unroll
+					for (int sb = 0; sb < C::SPB; sb++)
+						stage(st0 + sb, sb);
+			} else {
+				for (int st = 0; st < nk; st++)
+					stage(st, k0 + st);
 			}
 		} else {
-			lds_b<TYPE>(bbuf(0), bp, bi, k0, h, b);
-			prep(0, 0, 0);
-			for (int st = 0; st + 1 < nk; st++) {
-				steps(st, true);
+			lds_b<TYPE, DOWN, MTR>(bbuf(0), bp, bi, k0, h, b);
+			prep(0, k0, 0, 0);
+			auto stage = [&](int st, int sb) {
+				steps(st, sb, true);
 				// the last step's fragments are in registers: the barrier only
 				// waits for stage st + 1's data and this stage's LDS reads
 				barrier_after(st);
-				lds_b<TYPE>(bbuf(st + 1), bp, bi, k0 + st + 1, h, b);
+				lds_b<TYPE, DOWN, MTR>(bbuf(st + 1), bp, bi, sb + 1, h, b);
 				mm(L);
-				prep(st + 1, 0, L ^ 1);
+				prep(st + 1, sb + 1, 0, L ^ 1);
 				// order: the LDS reads, two MFMAs (their latency), then the
 				// preparation's VALU work spread between the other MFMAs
 				__builtin_amdgcn_sched_group_barrier(0x100, 32, 0);
@@ -1259,8 +1288,18 @@ __device__ __forceinline__ void run_tile(const MfmaArgs &a, uint8_t *As, uint32_
 					__builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
 				}
 				__builtin_amdgcn_sched_barrier(0);
+			};
+			if constexpr (C::RES) {
+				for (int st0 = 0; st0 < nk; st0 += C::SPB)
+#pragma unroll
+					for (int sb = 0; sb < C::SPB; sb++)
+						if (sb + 1 < C::SPB || st0 + C::SPB < nk)
+							stage(st0 + sb, sb);
+			} else {
+				for (int st = 0; st + 1 < nk; st++)
+					stage(st, k0 + st);
 			}
-			steps(nk - 1, false);
+			steps(nk - 1, C::RES ? C::SPB - 1 : k0 + nk - 1, false);
 			stage_barrier(); // every wave's LDS reads done before the epilogue reuses the buffers
 			mm(L);
 		}
