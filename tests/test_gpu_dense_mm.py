@@ -1,7 +1,8 @@
 """Dense products.  Exact ones of 5 and more tokens (the block dots on the fp32
 matrix cores), bit for bit against the oracle's rows: quads of tokens and
 their remainders, one and several groups, one super-block column and more
-than the workgroup's waves, both workgroup sizes, and inputs whose products
+than the workgroup's waves, both workgroup sizes (BF16 rows: pairs of tokens
+and a single one), and inputs whose products
 reach zeros of both signs, denormals and infinities.  Matrix-core ones on
 both sides of the K split and of each of its tile heights, down to one K
 stage per group, against a float64 model of their operands."""
@@ -26,7 +27,7 @@ def device():
     tie_amd.shutdown()
 
 
-@pytest.mark.parametrize("wtype", [synth.Q4_K, synth.Q6_K])
+@pytest.mark.parametrize("wtype", [synth.Q4_K, synth.Q6_K, synth.BF16])
 @pytest.mark.parametrize("rows,inn,T", [(64, 256, 5), (64, 512, 6), (128, 256, 7), (64, 768, 8), (64, 256, 9),
                                         (64, 512, 11), (64, 2304, 13), (4096, 256, 34)])
 def test_dense_exact_groups(wtype, rows, inn, T):
