@@ -29,7 +29,7 @@ def device():
 
 @pytest.mark.parametrize("wtype", [synth.Q4_K, synth.Q6_K, synth.BF16])
 @pytest.mark.parametrize("rows,inn,T", [(64, 256, 5), (64, 512, 6), (128, 256, 7), (64, 768, 8), (64, 256, 9),
-                                        (64, 512, 11), (64, 2304, 13), (4096, 256, 34)])
+                                        (64, 512, 11), (64, 2304, 13), (64, 8448, 9), (4096, 256, 34)])
 def test_dense_exact_groups(wtype, rows, inn, T):
     import torch
     rng = np.random.default_rng(17 + rows + inn + T + wtype)

@@ -32,7 +32,10 @@
 //                      (swiglu_activation_f32_f32_avx2) for its pairs in
 //                      LDS; the blocks then read h as LDS broadcasts.
 //   BF16 weights       two threads per row, each owning four of the row's
-//                      eight lane accumulators.
+//                      eight lane accumulators; inputs in LDS, two pairs per
+//                      pass over a row (bf16_row_dots).
+//   dense matrices     (launch_dense) the gate/up kernel per (panel, group of
+//                      8 tokens), its dots on the fp32 matrix cores.
 // No kernel waits on another workgroup: the only ordering is the launch
 // order on the stream.
 #include <cmath>

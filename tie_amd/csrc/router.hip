@@ -251,8 +251,8 @@ router_mm_kernel(const float *__restrict__ x, const float *__restrict__ WM, cons
 	const int net = E / (16 * NE), ntt = (T + TOK - 1) / TOK;
 	int tt, et;
 	if (by_token) {
-		tt = (int)(blockIdx.x / (8 * net)) * 8 + (int)(blockIdx.x % 8);
-		et = (int)(blockIdx.x / 8) % net;
+		tt = (int)((blockIdx.z * gridDim.y + blockIdx.y) * 8 + blockIdx.x % 8);
+		et = (int)blockIdx.x / 8;
 		if (tt >= ntt)
 			return;
 	} else {
@@ -497,8 +497,12 @@ hipError_t launch_router_logits(const Layer &L, const float *x, int T, float *lo
 			const int by_token = T >= 256 ? 1 : 0; // x the larger operand
 			if (conv)
 				conv->tiles = net;
-			tie_launch(kern, dim3(by_token ? (ntt + 7) / 8 * 8 * net : ntt * net), dim3(64 * RM_NW), 0, s, x,
-				   L.routerM, L.bias, T, d, E, logits, by_token, z, conv ? *conv : XConvArgs());
+			// 8 token tiles x all expert tiles in x, groups of 8 in y and z: one
+			// dimension of tokens times experts would pass the launch limit of 2^32
+			// threads at 2^33 logits (a dense matrix of very many rows)
+			const int n8 = (ntt + 7) / 8, y = n8 < 32768 ? n8 : 32768;
+			tie_launch(kern, by_token ? dim3(8 * net, y, (n8 + y - 1) / y) : dim3(ntt * net), dim3(64 * RM_NW),
+				   0, s, x, L.routerM, L.bias, T, d, E, logits, by_token, z, conv ? *conv : XConvArgs());
 		};
 		// larger tiles (fewer x transpositions and weight reads per MFMA) once
 		// they still cover most of the CUs: 30B T=500 (64 tiles of 32 x 32)
