@@ -851,6 +851,23 @@ extern "C" int tie_hip_moe_forward_noalloc(tie_hip_layer *layer, const float *x_
 // x of the host-buffer calls that go through pinned staging, at most (above,
 // the copies' bandwidth counts, not their latency)
 constexpr size_t PIN_MAX = (size_t)256 << 10;
+// (no memory to pin: false, and the call copies from the caller's buffers)
+static bool ensure_pin(size_t need)
+{
+	if (need <= g.pin_bytes)
+		return true;
+	if (g.pin)
+		(void)hipHostFree(g.pin); // (every call leaves the stream drained)
+	g.pin = nullptr;
+	g.pin_bytes = 0;
+	if (hipHostMalloc((void **)&g.pin, need, hipHostMallocMapped) != hipSuccess) {
+		(void)hipGetLastError();
+		g.pin = nullptr;
+		return false;
+	}
+	g.pin_bytes = need;
+	return true;
+}
 
 // The host-buffer drop-ins: the layer comes from the weight cache (uploaded
 // at the first call with these weights), x goes up, out and the selection
@@ -926,20 +943,12 @@ static int moe_ffn_host(const float *x, int T, int d, int F, int E, int k, const
 		g.io_k = nk;
 	}
 	const size_t nx = (size_t)T * d * 4, nk = (size_t)T * k * 4, nn = ffn_norm ? (size_t)d * 4 : 0;
-	if (nx <= PIN_MAX) {
+	const size_t ax = align256(nx), an = align256(nn), ak = align256(nk);
+	if (nx <= PIN_MAX && ensure_pin(2 * ax + an + 2 * ak)) {
 		// a few tokens: through pinned memory that the kernels read and write
 		// themselves (copies from and to pageable memory each hold the host
 		// until they are done: 30B T=1 with norm and selection 120 us a call,
 		// of which the kernels 28)
-		const size_t ax = align256(nx), an = align256(nn), ak = align256(nk), need = 2 * ax + an + 2 * ak;
-		if (need > g.pin_bytes) {
-			if (g.pin)
-				HIP_TRY(hipHostFree(g.pin)); // (every call leaves the stream drained)
-			g.pin = nullptr;
-			g.pin_bytes = 0;
-			HIP_TRY(hipHostMalloc((void **)&g.pin, need, hipHostMallocMapped));
-			g.pin_bytes = need;
-		}
 		uint8_t *hx = g.pin, *hn = hx + ax, *ho = hn + an, *hi = ho + ax, *hw = hi + ak;
 		memcpy(hx, x, nx);
 		if (nn)
