@@ -30,6 +30,7 @@ _NAMES = (
     ("tie::router_small_kernel", "router"),
     ("tie::router_mid_kernel", "router"),
     ("tie::router_logits_kernel", "router"),
+    ("tie::router_mm_kernel", "router"),
     ("tie::router_topk_kernel", "router"),
     ("tie::router_topk_wave_kernel", "router"),
     ("tie::route_group_kernel", "route_group"),
