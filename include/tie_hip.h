@@ -158,7 +158,8 @@ size_t tie_hip_layer_bytes(const tie_hip_layer *layer);
  *
  * Streams: the library keeps one scratch workspace per stream, so forwards
  * enqueued on different streams never share scratch memory and may run
- * concurrently (on distinct out buffers).  Forwards on one stream are
+ * concurrently (on distinct out buffers; the topk buffers are only written,
+ * so sharing them spoils them alone).  Forwards on one stream are
  * ordered by that stream.  When a call needs a larger workspace than its
  * stream holds, the library drains the whole device (hipDeviceSynchronize)
  * before freeing the old one; a call made during HIP graph capture must

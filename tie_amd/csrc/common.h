@@ -104,6 +104,15 @@ struct Layer {
 	size_t bytes = 0;
 };
 
+// The caller's copies of a forward's selection (each may be null): written
+// by the kernel that combines (the kernels before it read the workspace's
+// selection) and read by none, so that what other work does to the caller's
+// buffers meanwhile cannot reach this forward's results.
+struct SelOut {
+	int32_t *idx = nullptr; // [T][k]
+	float *w = nullptr;     // [T][k]
+};
+
 // Per-forward scratch (grown on demand, one per device).
 struct Workspace {
 	int32_t *topk_idx = nullptr;  // [T][k]
@@ -200,7 +209,7 @@ hipError_t launch_router_order(const Layer &L, hipStream_t s);
 hipError_t launch_dispatch(const Layer &L, int T, int k, const int32_t *topk_idx, Workspace &ws, hipStream_t s);
 hipError_t launch_route_group(const Layer &L, int T, int k, const float *logits, Workspace &ws, hipStream_t s);
 hipError_t launch_exact_block(const Layer &L, const float *x, int T, int k, const float *silu, Workspace &ws,
-			      float *out, hipStream_t s, const float *res = nullptr);
+			      float *out, hipStream_t s, const float *res, const SelOut &sel);
 hipError_t launch_mfma_experts(const Layer &L, const float *x, int T, int k, const float *silu, Workspace &ws,
 			       hipStream_t s);
 // True when the matrix-core path of this layer takes f16 operands, whose
@@ -223,11 +232,13 @@ hipError_t launch_recompute(const Layer &L, const float *x, int k, const float *
 bool combine_fix_preferred(const Layer &L);
 hipError_t launch_combine_fix(const Layer &L, const float *x, int k, const float *silu, const int32_t *topk_idx,
 			      const float *topk_w, const void *y, bool y16, int y_shift, float *out, const float *res,
-			      const int32_t *skip, const int32_t *list, const int32_t *count, int T, hipStream_t s);
+			      const int32_t *skip, const int32_t *list, const int32_t *count, int T, const SelOut &sel,
+			      hipStream_t s);
 
 hipError_t launch_decode(const Layer &L, const float *x, int k, const float *silu, const float *logits,
 			 int32_t *topk_idx, float *topk_w, float *h, float *out, const float *res, const int32_t *list,
-			 const int32_t *count, int max_entries, bool inline_route, bool fixup, hipStream_t s);
+			 const int32_t *count, int max_entries, bool inline_route, bool fixup, const SelOut &sel,
+			 hipStream_t s);
 // T = 1 in one launch (router, gate/up and down + combine workgroups that
 // hand the logits and h over as sequence-stamped words in lg / hw; E <= 128)
 bool decode_one_supported(const Layer &L, int k);
@@ -288,8 +299,8 @@ int dense_groups(int T);
 // res (optional): out = res + combine (the residual add after the block)
 // y16: y holds f16(y 2^-y_shift) (the matrix-core path's quantised down)
 hipError_t launch_combine(int T, int d, int k, const float *topk_w, const int32_t *topk_idx, const float *y,
-			  float *out, hipStream_t s, const float *res = nullptr, const int32_t *skip = nullptr,
-			  bool y16 = false, int y_shift = 0);
+			  float *out, hipStream_t s, const SelOut &sel, const float *res = nullptr,
+			  const int32_t *skip = nullptr, bool y16 = false, int y_shift = 0);
 // dst[i] = src[i] for up to three runs of 4-byte words, by one small kernel
 // (16-byte accesses where a run's pointers allow them): pinned host memory to
 // and from the device without the latency of a copy engine's commands
@@ -425,6 +436,21 @@ __device__ __forceinline__ float tie_swiglu(float g, float u, const float *__res
 	float s = __builtin_fmaf(frac, y2 - y1, y1);
 	return s * u;
 }
+// Token t's selection to the caller's copies, by the workgroup of the
+// token's first columns (at least 32 threads, as k <= 32).  After the
+// columns: a store before them takes the scalar loads from the selection
+// that the combine reads (30B T=64 4.0 -> 5.8 us).
+__device__ __forceinline__ void copy_selection(const SelOut &sel, int t, int k, const int32_t *__restrict__ topk_idx,
+					       const float *__restrict__ topk_w)
+{
+	if ((int)threadIdx.x < k) {
+		if (sel.idx)
+			sel.idx[(size_t)t * k + threadIdx.x] = topk_idx[(size_t)t * k + threadIdx.x];
+		if (sel.w)
+			sel.w[(size_t)t * k + threadIdx.x] = topk_w[(size_t)t * k + threadIdx.x];
+	}
+}
+
 // One token's combine over 8 columns (c8: 8-column group) of the expert
 // outputs: out[t][c] = [res[t][c] +] sum_j fma(g_j, y[t*k+j][c], .) in slot
 // order (model_qwen3.c:459-467, then the residual add of

@@ -511,6 +511,7 @@ struct DecodeArgs {
 	const int32_t *count;  // number of list entries (device)
 	int routing;
 	const float *pbias;
+	SelOut sel;            // the caller's copies of the selection
 };
 
 __device__ __forceinline__ int list_count(const DecodeArgs &a)
@@ -677,6 +678,8 @@ template <int TD> __global__ __launch_bounds__(DEC_MAX_THREADS) void decode_down
 		}
 		__syncthreads();
 		combine_rows(part, nb, k, R, sel_idx, sel_w, a.out + (size_t)t * a.d + r0, a.res ? a.res + (size_t)t * a.d + r0 : nullptr);
+		if (blockIdx.x == 0)
+			copy_selection(a.sel, t, k, a.topk_idx, a.topk_w);
 		__syncthreads();
 	}
 }
@@ -1229,12 +1232,16 @@ __global__ __launch_bounds__(CF_THREADS) void combine_fix_kernel(DecodeArgs a, C
 	const int t = b / c.cpt;
 	// 8 columns per thread, 16-byte loads of y (d is a multiple of 256)
 	const int c8 = (b - t * c.cpt) * CF_THREADS + threadIdx.x;
-	if (c.skip[t] || c8 * 8 >= a.d)
+	if (c8 * 8 >= a.d)
 		return;
-	if (c.y16)
-		combine8_cols<true>(t, c8, a.d, a.k, c.topk_w, c.topk_idx, c.y16, c.ysc, a.res, a.out);
-	else
-		combine8_cols<false>(t, c8, a.d, a.k, c.topk_w, c.topk_idx, c.y32, 1.0f, a.res, a.out);
+	if (!c.skip[t]) {
+		if (c.y16)
+			combine8_cols<true>(t, c8, a.d, a.k, c.topk_w, c.topk_idx, c.y16, c.ysc, a.res, a.out);
+		else
+			combine8_cols<false>(t, c8, a.d, a.k, c.topk_w, c.topk_idx, c.y32, 1.0f, a.res, a.out);
+	}
+	if (b == t * c.cpt)
+		copy_selection(a.sel, t, a.k, c.topk_idx, c.topk_w);
 }
 
 // ---------------------------------------------------------------- launchers
@@ -1298,8 +1305,7 @@ hipError_t launch_recompute(const Layer &L, const float *x, int k, const float *
 			    const float *topk_w, float *out, const float *res, const int32_t *list,
 			    const int32_t *count, int T, hipStream_t s)
 {
-	DecodeArgs a;
-	memset(&a, 0, sizeof a);
+	DecodeArgs a = {};
 	a.w[0] = L.gate.data;
 	a.w[1] = L.up.data;
 	a.w[2] = L.down.data;
@@ -1351,12 +1357,13 @@ bool combine_fix_preferred(const Layer &L)
 // alone) and the exact recomputation of the listed tokens, in one launch.
 hipError_t launch_combine_fix(const Layer &L, const float *x, int k, const float *silu, const int32_t *topk_idx,
 			      const float *topk_w, const void *y, bool y16, int y_shift, float *out, const float *res,
-			      const int32_t *skip, const int32_t *list, const int32_t *count, int T, hipStream_t s)
+			      const int32_t *skip, const int32_t *list, const int32_t *count, int T, const SelOut &sel,
+			      hipStream_t s)
 {
 	if (T == 0)
 		return hipSuccess;
-	DecodeArgs a;
-	memset(&a, 0, sizeof a);
+	DecodeArgs a = {};
+	a.sel = sel;
 	a.w[0] = L.gate.data;
 	a.w[1] = L.up.data;
 	a.w[2] = L.down.data;
@@ -1412,10 +1419,11 @@ hipError_t launch_combine_fix(const Layer &L, const float *x, int k, const float
 // dimension (entries beyond it are looped over).
 hipError_t launch_decode(const Layer &L, const float *x, int k, const float *silu, const float *logits,
 			 int32_t *topk_idx, float *topk_w, float *h, float *out, const float *res, const int32_t *list,
-			 const int32_t *count, int max_entries, bool inline_route, bool fixup, hipStream_t s)
+			 const int32_t *count, int max_entries, bool inline_route, bool fixup, const SelOut &sel,
+			 hipStream_t s)
 {
-	DecodeArgs a;
-	memset(&a, 0, sizeof a);
+	DecodeArgs a = {};
+	a.sel = sel;
 	a.w[0] = L.gate.data;
 	a.w[1] = L.up.data;
 	a.w[2] = L.down.data;

@@ -167,15 +167,19 @@ hipError_t launch_route_group(const Layer &L, int T, int k, const float *logits,
 // block (dispatch_apply_residual, model_qwen3.c:491, apply_residual_f32_f32_avx2
 // math_avx2.c:731-751).  res may be out (the hidden state updated in place).
 // Tokens with skip[t] != 0 (skip optional) are left alone: the exact
-// recomputation writes their rows afterwards, from res as it was.
+// recomputation writes their rows afterwards, from res as it was.  sel: the
+// caller's copies of the selection.
 __global__ __launch_bounds__(256) void combine_kernel(int T, int d, int k, const float *__restrict__ topk_w,
 						      const int32_t *__restrict__ topk_idx,
 						      const float *__restrict__ y, const float *res, float *out,
-						      const int32_t *__restrict__ skip)
+						      const int32_t *__restrict__ skip, SelOut sel)
 {
 	const int t = blockIdx.y;
-	if (skip && skip[t])
+	if (skip && skip[t]) {
+		if (blockIdx.x == 0)
+			copy_selection(sel, t, k, topk_idx, topk_w);
 		return;
+	}
 	const int c4 = blockIdx.x * blockDim.x + threadIdx.x; // float4 column
 	if (c4 * 4 >= d)
 		return;
@@ -216,25 +220,34 @@ __global__ __launch_bounds__(256) void combine_kernel(int T, int d, int k, const
 		acc.w = h.w + acc.w;
 	}
 	reinterpret_cast<float4 *>(out + (size_t)t * d)[c4] = acc;
+	if (blockIdx.x == 0)
+		copy_selection(sel, t, k, topk_idx, topk_w);
 }
 
 // The same with 8 columns per thread for f16 y scaled by 2^-y_shift (the
 // matrix-core path's quantised down; combine8_cols)
 __global__ __launch_bounds__(256) void combine16_kernel(int T, int d, int k, const float *__restrict__ topk_w,
 							const int32_t *__restrict__ topk_idx, const uint16_t *__restrict__ y,
-							float ysc, const float *res, float *out, const int32_t *__restrict__ skip)
+							float ysc, const float *res, float *out, const int32_t *__restrict__ skip,
+							SelOut sel)
 {
 	const int t = blockIdx.y;
-	if (skip && skip[t])
+	if (skip && skip[t]) {
+		if (blockIdx.x == 0)
+			copy_selection(sel, t, k, topk_idx, topk_w);
 		return;
+	}
 	const int c8 = blockIdx.x * blockDim.x + threadIdx.x;
 	if (c8 * 8 >= d)
 		return;
 	combine8_cols<true>(t, c8, d, k, topk_w, topk_idx, y, ysc, res, out);
+	if (blockIdx.x == 0)
+		copy_selection(sel, t, k, topk_idx, topk_w);
 }
 
 hipError_t launch_combine(int T, int d, int k, const float *topk_w, const int32_t *topk_idx, const float *y,
-			  float *out, hipStream_t s, const float *res, const int32_t *skip, bool y16, int y_shift)
+			  float *out, hipStream_t s, const SelOut &sel, const float *res, const int32_t *skip, bool y16,
+			  int y_shift)
 {
 	if (T == 0)
 		return hipSuccess;
@@ -242,12 +255,12 @@ hipError_t launch_combine(int T, int d, int k, const float *topk_w, const int32_
 		if (d % 8)
 			return hipErrorInvalidValue;
 		tie_launch(combine16_kernel, dim3((d / 8 + 255) / 256, T), dim3(256), 0, s, T, d, k, topk_w, topk_idx,
-			   reinterpret_cast<const uint16_t *>(y), ldexpf(1.0f, y_shift), res, out, skip);
+			   reinterpret_cast<const uint16_t *>(y), ldexpf(1.0f, y_shift), res, out, skip, sel);
 		return hipGetLastError();
 	}
 	const int n4 = d / 4;
 	tie_launch(combine_kernel, dim3((n4 + 255) / 256, T), dim3(256), 0, s, T, d, k, topk_w, topk_idx, y, res,
-			   out, skip);
+			   out, skip, sel);
 	return hipGetLastError();
 }
 
