@@ -305,11 +305,24 @@ template <int TYPE, bool DOWN = false, int MTR = 0> struct Cfg {
 	// loads in flight); the stage loops are unrolled by the block, so the
 	// sub-block arithmetic of the scales is constant too.  Read again in every
 	// stage, these chunks were a third of Q6_K's L2-to-LDS bytes and a quarter
-	// of Q4_K's.  Kernels, one box, without / with: down (Q6_K) 30B T=32 34.9 /
-	// 32.8 us, T=101 41.4 / 39.0, T=500 52.8 / 47.5, T=2048 104.7 / 97.0, 235B
-	// T=1024 208 / 190; gate/up (Q4_K) T=32 43.8 / 42.2, T=256 56.2 / 51.7,
-	// T=2048 147.7 / 146.4, 235B T=1024 304 / 292; Q4_K down T=500 41.5 / 39.3
+	// of Q4_K's.  Kernels, without / with (same weight DMA order, one card):
+	// down Q6_K 30B T=32 35.8 / 33.4 us, T=101 42.4 / 40.2, T=500 52.6 / 49.5,
+	// T=2048 100 / 94, 235B T=1024 202 / 185; gate/up Q4_K 32-row tiles T=32
+	// 42.9 / 41.1, T=64 48.4 / 44.4; Q6_K T=64 63.7 / 62.4; 64-row tiles
+	// Q4_K 30B T=500 65.6 / 67.2 (d = 2048), 235B T=1024 300 / 284, Q6_K
+	// T=500 99 / 89; 160-row tiles Q4_K T=2048 126 / 127, Q6_K 186 / 179 (the
+	// Q6_K 32- and 160-row gate/up kernels are ahead although they spill 1 and
+	// 3 registers with it; Q4_K's 160-row one spills 1 either way).
 	static constexpr bool RES = F16 && KST == 64 && KS == 1 && NS == 2 && QK / KST == 4;
+	// The waves of a workgroup take a weight stage's chunks in turn, panel by
+	// panel (dma_b), instead of a panel each: the four waves' loads then cover
+	// a few KiB of one or two panels at a time, not the same chunk of four
+	// panels some 72 KiB apart.  The gate/up kernels of decode-sized batches,
+	// bound by the weight stream, gain by it: 30B Q4_K T=64 43.4 us, a panel
+	// each 44.1, Q6_K 62.4 / 66.6; on a card with slower memory (without RES)
+	// 49.8 / 55.4.  Down and the larger tiles do not: 30B T=2048 down 94.1 us
+	// with a panel each, 96.3 in turn.
+	static constexpr bool IN_TURN = !SPLIT && !DOWN && MTR == MFMA_MT_TINY;
 	// DMA instructions one wave issues per weight stage (dma_b)
 	static constexpr int B_DMA = NCH + (TYPE == TIE_GGML_Q6_K ? 1 : 0);
 	static constexpr int LDS_A = NS * ABUF, LDS_B = B_LDS ? NS * BBUF : 0;
@@ -384,22 +397,26 @@ __device__ __forceinline__ void load_b(const BSrc &s, int st, int h, BRegs<TYPE>
 // stage's ql chunks, 2, 3 the block half's qh chunks, 4 the scales; then the 4
 // panels' d planes (128 B each).  Parts that a block's later stages use too
 // are moved once (Cfg::RES).
-// Wave w moves panel w's chunks; their base and panel offset are set once per
-// tile (BDma).
+// Wave w moves panel w's chunks, or (Cfg::IN_TURN) every fourth of the four
+// panels' chunks.
 struct BDma {
-	const uint8_t *base; // expert base of panel w's matrix (wave-uniform)
-	uint32_t pofs;       // the panel row's offset in the expert (wave-uniform)
+	const uint8_t *base; // expert base of panel w's matrix (IN_TURN: gate's)
+	const uint8_t *up;   // IN_TURN: expert base of up
+	uint32_t pofs;       // panel w's row offset in the expert (IN_TURN: panel 0's)
+	uint32_t pstride;    // from a panel row to the next
 	uint32_t lane16;     // 16 * lane
 };
 
-template <int TYPE, bool DOWN>
+template <int TYPE, bool DOWN, int MTR>
 __device__ __forceinline__ void bdma_init(const MfmaArgs &a, int e, int slab, int w, BDma &d)
 {
-	const int mat = DOWN ? 0 : w >> 1;
-	const int rt = DOWN ? 4 * slab + w : 2 * slab + (w & 1);
-	d.base = a.w[mat] + (size_t)e * a.expert_bytes[mat];
-	d.pofs = (uint32_t)rt * (uint32_t)(a.in / QK) * (uint32_t)panel_bytes(TYPE);
+	d.pstride = (uint32_t)(a.in / QK) * (uint32_t)panel_bytes(TYPE);
 	d.lane16 = 16u * (threadIdx.x & 63);
+	const int p = Cfg<TYPE, DOWN, MTR>::IN_TURN ? 0 : w;
+	const int mat = DOWN ? 0 : p >> 1;
+	d.base = a.w[mat] + (size_t)e * a.expert_bytes[mat];
+	d.up = a.w[1] + (size_t)e * a.expert_bytes[1];
+	d.pofs = (uint32_t)(DOWN ? 4 * slab + p : 2 * slab + (p & 1)) * d.pstride;
 }
 
 // Whether stage st (mod the stages per block) reads slot c of a panel from
@@ -420,27 +437,44 @@ __device__ __forceinline__ void dma_b(const BDma &d, int st, int sb, int w, uint
 	using C = Cfg<TYPE, DOWN, MTR>;
 	const int half = sb & 1, part = sb % C::SPB;
 	const uint32_t kofs = (uint32_t)(st / C::SPB) * (uint32_t)panel_bytes(TYPE);
-	const uint32_t lb = lds_addr(B) + w * C::PB;
-#pragma unroll
-	for (int s = 0; s < C::NCH; s++) {
-		if (!slot_moved<TYPE, C>(sb, s))
-			continue;
-		int chunk;
+	auto chunk_of = [&](int s) {
 		if constexpr (TYPE == TIE_GGML_Q4_K)
-			chunk = s == 0 ? 0 : (C::NCH - 1) * part + s;
+			return s == 0 ? 0 : (C::NCH - 1) * part + s;
 		else if constexpr (C::APERM) {
 			// ql chunks of quarters q, q + 2 of half n; the half's qh; scales
 			const int n = (sb >> 1) & 1, q = sb & 1;
-			chunk = s < 2 ? 4 * n + 2 * q + s : (s < 4 ? 8 + 2 * n + (s - 2) : 12);
+			return s < 2 ? 4 * n + 2 * q + s : (s < 4 ? 8 + 2 * n + (s - 2) : 12);
 		} else
-			chunk = s < 4 ? 4 * half + s : (s < 6 ? 8 + 2 * half + (s - 4) : 12);
-		dma16s(d.base, d.lane16 + (d.pofs + kofs + (uint32_t)chunk * 1024),
-		       __builtin_amdgcn_readfirstlane(lb + s * 1024));
+			return s < 4 ? 4 * half + s : (s < 6 ? 8 + 2 * half + (s - 4) : 12);
+	};
+	if constexpr (C::IN_TURN) {
+		int first = C::NCH, n = 0; // the stage moves slots first .. first + n - 1
+#pragma unroll
+		for (int s = 0; s < C::NCH; s++)
+			if (slot_moved<TYPE, C>(sb, s)) {
+				first = s < first ? s : first;
+				n++;
+			}
+#pragma unroll
+		for (int c = 0; c < C::NCH; c++) {
+			if (c >= n)
+				break;
+			const int it = NWAVES * c + w, p = it / n, s = first + it - p * n; // 4 n items: p < 4
+			dma16s(p > 1 ? d.up : d.base, d.lane16 + (d.pofs + (p & 1) * d.pstride + kofs + (uint32_t)chunk_of(s) * 1024),
+			       __builtin_amdgcn_readfirstlane(lds_addr(B) + p * C::PB + s * 1024));
+		}
+	} else {
+#pragma unroll
+		for (int s = 0; s < C::NCH; s++)
+			if (slot_moved<TYPE, C>(sb, s))
+				dma16s(d.base, d.lane16 + (d.pofs + kofs + (uint32_t)chunk_of(s) * 1024),
+				       __builtin_amdgcn_readfirstlane(lds_addr(B) + w * C::PB + s * 1024));
 	}
 	if constexpr (TYPE == TIE_GGML_Q6_K) {
 		// the d plane of panel w (128 B)
 		if (slot_moved<TYPE, C>(sb, -1) && (threadIdx.x & 63) < 8)
-			dma16s(d.base, d.lane16 + (d.pofs + kofs + Q6K_CHUNKS * 1024),
+			dma16s(C::IN_TURN && w > 1 ? d.up : d.base,
+			       d.lane16 + (d.pofs + (C::IN_TURN ? (w & 1) * d.pstride : 0u) + kofs + Q6K_CHUNKS * 1024),
 			       __builtin_amdgcn_readfirstlane(lds_addr(B) + 4 * C::PB + w * 128));
 	}
 }
@@ -1107,7 +1141,7 @@ __device__ __forceinline__ void run_tile(const MfmaArgs &a, uint8_t *As, uint32_
 		constexpr int NA = NMT;
 		static_assert(C::NPL == 1 && C::NSTEP % 2 == 0, "one activation plane, even step count");
 		BDma bd;
-		bdma_init<TYPE, DOWN>(a, e, slab, w, bd);
+		bdma_init<TYPE, DOWN, MTR>(a, e, slab, w, bd);
 		constexpr int NS = C::NS;
 		auto abuf = [&](int st) { return As + (st % NS) * C::ABUF; };
 		auto bbuf = [&](int st) { return Bs + (st % NS) * C::BBUF; };
