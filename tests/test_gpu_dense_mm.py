@@ -4,8 +4,8 @@ their remainders, one and several groups, one super-block column and more
 than the workgroup's waves, both workgroup sizes (BF16 rows: pairs of tokens
 and a single one), and inputs whose products
 reach zeros of both signs, denormals and infinities.  Matrix-core ones on
-both sides of the K split and of each of its tile heights, down to one K
-stage per group, against a float64 model of their operands."""
+both sides of the K split (by the inputs, 512 and 768, and by the workgroups)
+and of each of its tile heights, against a float64 model of their operands."""
 import numpy as np
 import pytest
 
@@ -49,11 +49,12 @@ def test_dense_exact_groups(wtype, rows, inn, T):
     np.testing.assert_array_equal(bits(got)[~nan], bits(ref)[~nan])
 
 
-# one workgroup per CU or fewer (32-, 64- and 128-row tiles with their K
-# groups; 4 stages of 64 in all, then an odd number per block), and more
+# one workgroup per CU or fewer (32-, 64- and 128-row tiles, whole up to 512
+# inputs, with their K groups from 768 on), and more
 @pytest.mark.parametrize("wtype", [synth.Q4_K, synth.Q6_K])
 @pytest.mark.parametrize("rows,inn,T", [(256, 256, 1), (512, 768, 33), (4096, 256, 512), (4096, 256, 1021),
-                                        (4096, 512, 2047), (4096, 256, 2049)])
+                                        (4096, 512, 2047), (4096, 256, 2049), (4096, 768, 509), (4096, 768, 1021),
+                                        (4096, 768, 2048), (4096, 768, 2049)])
 def test_dense_mfma_k_groups(wtype, rows, inn, T):
     import torch
     rng = np.random.default_rng(29 + rows + inn + T + wtype)

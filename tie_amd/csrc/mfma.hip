@@ -2389,14 +2389,20 @@ hipError_t launch_mfma_dense(const ExpertTensor &W, const float *x, int T, float
 	a.dense_t = T;
 	// one workgroup per CU or fewer: their 4 waves alone leave each SIMD's
 	// dequantisation, LDS reads and MFMAs in series, so the K stages go to 2
-	// or 4 groups of waves per workgroup (as many as the LDS and registers
-	// hold).  Q4_K 4096 x 2048: T=509 26.6 -> 22.5 us, T=1000 34.3 -> 29.2,
-	// T=2000 46.3 -> 41.2; Q6_K 4096 x 4096: T=500 59.1 -> 52, T=2048 96.9 ->
-	// 84.  With more workgroups than CUs two share each anyway (Q4_K 6144 x
-	// 2048, T=900: 45.5 us, split 49.4).  More stage buffers instead of the
-	// split: no gain (Q6_K 10% slower).
+	// or 4 groups of waves per workgroup (as many as the LDS holds; by the
+	// registers the 32-row Q4_K kernel spills 8 and the 128-row ones 12, and
+	// they are faster all the same).  The whole product with its two other
+	// launches, Q4_K 4096 x 2048: T=509 32.6 -> 27.6 us, T=1000 38.4 -> 34.5,
+	// T=2048 54.4 -> 51.8; Q6_K 4096 x 2048: T=509 36.9 -> 32.4, T=2048 59.7
+	// -> 56.3.  With more workgroups than CUs two share each anyway (Q4_K 6144
+	// x 2048, T=900: 45.5 us, split 49.4).  Up to 512 inputs (8 stages in all)
+	// adding the groups' sums costs what the split gains: 4096 x 256, T=509
+	// Q4_K 12.8 us, split 14.3; 4096 x 512, T=2048 27.3 / 27.9 and Q6_K 28.0 /
+	// 29.2; from 768 inputs on it does not (T=2048 32.2 / 32.5, T=64 14.7 /
+	// 14.5).  More stage buffers instead of the split: no gain (Q6_K 10%
+	// slower).
 	const int q4 = W.type == TIE_GGML_Q4_K;
-	if (slabs * ((T + mt - 1) / mt) > 256)
+	if (slabs * ((T + mt - 1) / mt) > 256 || W.in <= 512)
 		err = launch_one<true>(a, W.type, grid, s);
 	else if (mt == 32)
 		err = q4 ? launch_type<TIE_GGML_Q4_K, true, mfma_ks(4) | 32>(a, grid, s)
