@@ -297,8 +297,9 @@ void tie_hip_debug_decode_form(int form);
  * upload from samples of the gate and down weights. */
 int tie_hip_debug_layer_shifts(const tie_hip_layer *layer, int *h_shift, int *y_shift);
 
-/* Make the n-th next device allocation fail with TIE_HIP_ENOMEM (n >= 1;
- * 0 disarms).  Host-side fault injection for error-path tests. */
+/* Make the n-th next allocation fail (n >= 1; 0 disarms): of device memory
+ * with TIE_HIP_ENOMEM, of pinned host memory so that the call does without.
+ * Host-side fault injection for error-path tests. */
 void tie_hip_debug_fail_alloc(int n);
 
 /* Per-kernel timing: while enabled, every kernel of a named section (router,

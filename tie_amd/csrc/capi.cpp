@@ -184,6 +184,20 @@ static int dev_malloc(void **p, size_t bytes, const char *what)
 	return TIE_HIP_OK;
 }
 
+// Pinned host memory that the kernels read and write; null where there is
+// none to be had (the callers then do without it).
+static void *pin_malloc(size_t bytes)
+{
+	void *p = nullptr;
+	if (g_fail_alloc > 0 && --g_fail_alloc == 0)
+		return nullptr;
+	if (hipHostMalloc(&p, bytes, hipHostMallocMapped) != hipSuccess) {
+		(void)hipGetLastError();
+		return nullptr;
+	}
+	return p;
+}
+
 static size_t align256(size_t n)
 {
 	return (n + 255) & ~(size_t)255;
@@ -301,17 +315,12 @@ static int ensure_workspace(hipStream_t s, int T, int k, int d, int F, int E, Wo
 	const size_t EE = (size_t)E > w.cap_E ? E : w.cap_E;
 	const size_t bytes = carve_workspace(nullptr, P, FF, DD, EE, nullptr);
 	void *mem = nullptr;
-	int32_t *status = w.one_status; // (a given-up wait not yet reported survives the growth)
-	if (!status) {
-		HIP_TRY(hipHostMalloc((void **)&status, 64, hipHostMallocMapped));
-		*status = 0;
-		w.one_status = status;
-	}
 	if (w.alloc) {
 		// work still queued on s (or, through events, on any stream the
 		// caller chained to it) may read the old buffer: drain the device
 		HIP_TRY(hipDeviceSynchronize());
 		HIP_TRY(hipFree(w.alloc));
+		int32_t *status = w.one_status; // (a given-up wait not yet reported survives the growth)
 		w = Workspace();
 		w.one_status = status;
 	}
@@ -327,17 +336,29 @@ static int ensure_workspace(hipStream_t s, int T, int k, int d, int F, int E, Wo
 	return TIE_HIP_OK;
 }
 
+// The one-launch decode's status word of a workspace, at its first such
+// call; null without memory to pin (the call then takes the other kernels)
+static int32_t *ensure_status(Workspace &w)
+{
+	if (!w.one_status) {
+		w.one_status = (int32_t *)pin_malloc(64);
+		if (w.one_status)
+			*w.one_status = 0;
+	}
+	return w.one_status;
+}
+
 // The status word of stream s's workspace: TIE_HIP_EHIP (and the word
 // cleared) when a one-launch decode wait gave up since the last check.
 // Synchronises s.
 static int take_stream_status(hipStream_t s)
 {
 	auto it = g.ws.find(s);
-	if (it == g.ws.end() || !it->second.one_status)
+	if (it == g.ws.end() || !it->second.alloc)
 		return TIE_HIP_OK;
 	HIP_TRY(hipStreamSynchronize(s));
 	volatile int32_t *st = it->second.one_status;
-	if (!*st)
+	if (!st || !*st)
 		return TIE_HIP_OK;
 	*st = 0;
 	return set_error(TIE_HIP_EHIP, "one-token forward: a wait between workgroups gave up (the GPU did not run "
@@ -555,7 +576,7 @@ static int forward(tie_hip_layer *layer, const float *x, int T, int k, float *ou
 	// one token, one launch (eager calls on a workspace of their own: the
 	// sequence number lives on the host, so a captured graph could not
 	// advance it)
-	const bool one = !mfma && T == 1 && !preset && !capturing(s) && decode_one_supported(L, k);
+	const bool one = !mfma && T == 1 && !preset && !capturing(s) && decode_one_supported(L, k) && ensure_status(ws);
 	if (norm && !(one && decode_one_norm_supported(L, k))) {
 		// (the one-launch kernel normalises its token itself)
 		prof_begin("rmsnorm", s);
@@ -874,13 +895,9 @@ static bool ensure_pin(size_t need)
 		(void)hipHostFree(g.pin); // (every call leaves the stream drained)
 	g.pin = nullptr;
 	g.pin_bytes = 0;
-	if (hipHostMalloc((void **)&g.pin, need, hipHostMallocMapped) != hipSuccess) {
-		(void)hipGetLastError();
-		g.pin = nullptr;
-		return false;
-	}
-	g.pin_bytes = need;
-	return true;
+	g.pin = (uint8_t *)pin_malloc(need);
+	g.pin_bytes = g.pin ? need : 0;
+	return g.pin != nullptr;
 }
 
 // The host-buffer drop-ins: the layer comes from the weight cache (uploaded
