@@ -49,6 +49,39 @@ def test_dense_exact_groups(wtype, rows, inn, T):
     np.testing.assert_array_equal(bits(got)[~nan], bits(ref)[~nan])
 
 
+@pytest.mark.parametrize("wtype", [synth.Q4_K, synth.Q6_K])
+def test_dense_exact_needs_no_scratch(wtype):
+    """The quantised exact products take no memory: the first call on a
+    stream, larger ones and one captured into a graph, with an allocation
+    failure armed all along."""
+    import torch
+    rows, inn = 64, 512
+    w = synth.expert_tensor(np.random.default_rng(41 + wtype), wtype, 1, rows, inn)
+    m = tie_amd.Matrix(w, wtype, rows, inn)
+    s = torch.cuda.Stream()
+    xs = {T: synth.make_input(42 + T, T, inn) for T in (5, 70)}
+    dev = {T: (torch.from_numpy(x).cuda(), torch.empty((T, rows), device="cuda")) for T, x in xs.items()}
+    torch.cuda.synchronize()
+    tie_amd.lib().tie_hip_debug_fail_alloc(1)
+    try:
+        for T in (5, 70):
+            m.mat_mat(dev[T][0], T, dev[T][1], stream=s.cuda_stream)
+        s.synchronize()
+        for T in (5, 70):
+            np.testing.assert_array_equal(bits(dev[T][1].cpu().numpy()), bits(bind.mat_mat(xs[T], w, wtype, rows)))
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            m.mat_mat(dev[70][0], 70, dev[70][1], stream=torch.cuda.current_stream().cuda_stream)
+        for _ in range(3):
+            dev[70][1].fill_(np.nan)
+            g.replay()
+            torch.cuda.synchronize()
+            np.testing.assert_array_equal(bits(dev[70][1].cpu().numpy()), bits(bind.mat_mat(xs[70], w, wtype, rows)))
+    finally:
+        tie_amd.lib().tie_hip_debug_fail_alloc(0)
+    m.close()
+
+
 # one workgroup per CU or fewer (32-, 64- and 128-row tiles, whole up to 512
 # inputs, with their K groups from 768 on), and more
 @pytest.mark.parametrize("wtype", [synth.Q4_K, synth.Q6_K])

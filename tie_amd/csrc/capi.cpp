@@ -1260,12 +1260,10 @@ extern "C" int tie_hip_mat_mat(tie_hip_matrix *m, const float *x_dev, int T, flo
 	} else if (dense_rows_supported(m->W, T)) {
 		HIP_TRY(launch_dense_rows(m->W, x_dev, T, out_dev, s));
 	} else {
-		const int G = dense_groups(T);
-		Workspace *ws = nullptr;
-		rc = ensure_workspace(s, T, 1, m->W.in, QK, G, &ws);
-		if (rc)
+		Workspace *ws = nullptr; // (the BF16 kernel's group lists)
+		if (m->W.type == TIE_GGML_BF16 && (rc = ensure_workspace(s, T, 1, m->W.in, QK, dense_groups(T), &ws)))
 			return rc;
-		HIP_TRY(launch_dense(m->W, x_dev, T, out_dev, *ws, s));
+		HIP_TRY(launch_dense(m->W, x_dev, T, out_dev, ws, s));
 	}
 	prof_end(s);
 	return TIE_HIP_OK;

@@ -279,9 +279,9 @@ struct Layer;
 int mfma_gu_rows(const Layer &L, int npairs); // rows per gate/up tile (the tile list's and the kernel's)
 int mfma_dn_rows(const Layer &L, int npairs); // rows per down tile
 // Dense F32-input matrix product through the expert GEMV kernels: out[t][r]
-// = W[r] . x[t] (W one "expert": rows, in, panel layout); dense_groups(T)
-// token groups (the workspace needs that many experts and T pairs)
-hipError_t launch_dense(const ExpertTensor &W, const float *x, int T, float *out, Workspace &ws, hipStream_t s);
+// = W[r] . x[t] (W one "expert": rows, in, panel layout).  BF16 needs a
+// workspace of T pairs and dense_groups(T) experts, the other types none.
+hipError_t launch_dense(const ExpertTensor &W, const float *x, int T, float *out, Workspace *ws, hipStream_t s);
 // The same for a few tokens (T <= 4, Q4_K / Q6_K): a lane per (row, block),
 // the block loaded once for all tokens (decode.hip); needs no workspace
 bool dense_rows_supported(const ExpertTensor &W, int T);

@@ -704,7 +704,6 @@ struct ExactArgs {
 	int32_t *offsets, *pairs, *active; // grouping (global)
 	int pg_cap;           // pairs per LDS group
 	int inline_route;
-	int dense;            // pairs are the tokens in order, slot s those from s * DENSE_GROUP on (no lists)
 	int single;           // T = 1 mode: slot j = pair j of expert topk_idx[j], no grouping
 	int routing;          // ROUTE_SOFTMAX / ROUTE_SIGMOID (inline routing)
 	const float *pbias;   // [E] selection bias of ROUTE_SIGMOID, or null
@@ -773,17 +772,21 @@ template <int NT> __device__ __forceinline__ void inline_route(const ExactArgs &
 // column w, w + 8, ..) and applies TIE's table SwiGLU
 // (swiglu_activation_f32_f32_avx2) to the row sums, writing h; otherwise
 // blockIdx.z selects the matrix and the row sums are written.
+// PM = MM_PAIRS: a dense matrix (launch_dense), one "expert" whose pairs are
+// the T tokens in order, slot s those from s * DENSE_GROUP on (no lists, no
+// routing), its dots on the matrix cores.
 template <int TYPE, bool FUSED, int PM>
 __global__ __launch_bounds__(GU_THREADS) GU_OCC void exact_gu_kernel(ExactArgs a)
 {
-	// fused: as many waves as the launch chose; split: GU_WAVES
-	const int NW = FUSED || PM == MM_PAIRS ? __builtin_amdgcn_readfirstlane(blockDim.x >> 6) : GU_WAVES;
+	constexpr bool DENSE = PM == MM_PAIRS;
+	// fused and dense: as many waves as the launch chose; else GU_WAVES
+	const int NW = FUSED || DENSE ? __builtin_amdgcn_readfirstlane(blockDim.x >> 6) : GU_WAVES;
 	using Block = typename BlockOf<TYPE>::type;
 	extern __shared__ float part[]; // [mats][nb][pg_cap][64]
 	const int32_t *offsets = a.offsets, *pairs = a.pairs, *active = a.active;
 	const int32_t *sel_idx = nullptr;
-	if constexpr (!FUSED) {
-		// the fused kernel never routes inline: no LDS reserved for it
+	if constexpr (!FUSED && !DENSE) {
+		// these kernels never route inline: no LDS reserved for it
 		__shared__ InlineRoute R;
 		if (a.inline_route) {
 			inline_route<GU_THREADS>(a, R);
@@ -796,17 +799,17 @@ __global__ __launch_bounds__(GU_THREADS) GU_OCC void exact_gu_kernel(ExactArgs a
 	auto single_expert = [&](const ExactArgs &, const int32_t *, int j) { return j < a.k ? sel_idx[j] : -1; };
 	const int slot = blockIdx.y;
 	int e, p0, p1;
-	if (!FUSED && a.single) {
+	if constexpr (DENSE) {
+		e = 0;
+		p0 = slot * DENSE_GROUP;
+		p1 = min(p0 + DENSE_GROUP, a.T);
+	} else if (!FUSED && a.single) {
 		// one token: the slot's selected expert, the slot's own pair
 		e = __builtin_amdgcn_readfirstlane(single_expert(a, pairs, slot));
 		if (e < 0)
 			return;
 		p0 = slot;
 		p1 = slot + 1;
-	} else if (PM == MM_PAIRS && a.dense) {
-		e = 0;
-		p0 = slot * DENSE_GROUP;
-		p1 = min(p0 + DENSE_GROUP, a.T);
 	} else {
 		if (slot >= active[a.E])
 			return;
@@ -827,7 +830,8 @@ __global__ __launch_bounds__(GU_THREADS) GU_OCC void exact_gu_kernel(ExactArgs a
 
 	for (int g0 = p0; g0 < p1; g0 += pg_cap) {
 		const int np = min(pg_cap, p1 - g0);
-		const int32_t *gp = pairs + g0;
+		// pair q of the group
+		auto pair_of = [&](int q) { return DENSE ? g0 + q : pairs[g0 + q]; };
 		const int ntask = nmat * nb;
 		auto panel_of = [&](int t) {
 			const int mi = t / nb, b = t - mi * nb;
@@ -838,13 +842,11 @@ __global__ __launch_bounds__(GU_THREADS) GU_OCC void exact_gu_kernel(ExactArgs a
 			Block blk;
 			load_block(panel_of(t), lane, blk);
 			auto xrow_b = [&](int q) {
-				const int pair = __builtin_amdgcn_readfirstlane(PM == MM_PAIRS && a.dense ? g0 + q : gp[q]);
+				const int pair = __builtin_amdgcn_readfirstlane(pair_of(q));
 				return (cfloat *)(x + (size_t)(pair / k) * in + QK * b);
 			};
-			if constexpr (PM == MM_PAIRS) {
-				auto xrow_v = [&](int q) {
-					return x + (size_t)(a.dense ? g0 + q : gp[q] / k) * in + QK * b;
-				};
+			if constexpr (DENSE) {
+				auto xrow_v = [&](int q) { return x + (size_t)pair_of(q) * in + QK * b; };
 				float *part_t = part + (size_t)t * pg_cap * 64;
 				if constexpr (TYPE == TIE_GGML_Q4_K) {
 					if (np > 4)
@@ -870,7 +872,7 @@ __global__ __launch_bounds__(GU_THREADS) GU_OCC void exact_gu_kernel(ExactArgs a
 		// serial sums over super-blocks (math_avx2.c:762-766)
 		for (int i = threadIdx.x; i < np * 64; i += 64 * NW) {
 			const int q = i >> 6, r = i & 63;
-			const size_t o = (size_t)(PM == MM_PAIRS && a.dense ? g0 + q : gp[q]) * a.rows + rt * PANEL_ROWS + r;
+			const size_t o = (size_t)pair_of(q) * a.rows + rt * PANEL_ROWS + r;
 			float s0 = 0.0f;
 			for (int b = 0; b < nb; b++)
 				s0 = s0 + part[((size_t)b * pg_cap + q) * 64 + r];
@@ -1238,7 +1240,7 @@ static hipError_t launch_gu_q(int type, bool fused, int nmat, int rows, int in, 
 	const size_t lds = sizeof(float) * (size_t)mats * nb * g.pg_cap * 64;
 	const dim3 grid(rows / PANEL_ROWS, max_active, fused ? 1 : nmat);
 	dim3 block(64 * GU_WAVES);
-	const size_t st = fused ? 0 : sizeof(InlineRoute);
+	const size_t st = fused || mm ? 0 : sizeof(InlineRoute);
 	constexpr int PM = TIE_EXACT_PCMAX;
 	// one token (one pair per group): a one-pair instance, whose register
 	// budget, and so occupancy, is not set by the multi-pair dot products
@@ -1444,11 +1446,12 @@ hipError_t launch_exact_block(const Layer &L, const float *x, int T, int k, cons
 // ------------------------------------------------------------ dense
 // dispatch_mat_mat (math_dispatch.c:304-359) with F32 input: every token row
 // through the same row kernel as the experts (mat_vec_row_f32_{q4k,q6k,
-// bf16}_f32_avx2), so the expert GEMV kernels run it unchanged: the tokens
-// are split into groups of DENSE_GROUP, and each group is an "expert" of
-// stride 0 (every group reads the one matrix), so groups spread over the
-// grid's y dimension and each workgroup computes one 64-row panel for one
-// group.  out[t][r], [T][rows].
+// bf16}_f32_avx2), by the expert GEMV kernels: the tokens are split into
+// groups of DENSE_GROUP, which spread over the grid's y dimension, so that
+// each workgroup computes one 64-row panel for one group.  The quantised
+// kernels know the groups (MM_PAIRS); the BF16 one reads them from lists, as
+// "experts" of stride 0 (every group reads the one matrix).  out[t][r],
+// [T][rows].
 __global__ void dense_groups_kernel(int T, int G, int32_t *offsets, int32_t *pairs, int32_t *active)
 {
 	const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1465,7 +1468,7 @@ int dense_groups(int T)
 	return (T + DENSE_GROUP - 1) / DENSE_GROUP;
 }
 
-hipError_t launch_dense(const ExpertTensor &W, const float *x, int T, float *out, Workspace &ws, hipStream_t s)
+hipError_t launch_dense(const ExpertTensor &W, const float *x, int T, float *out, Workspace *ws, hipStream_t s)
 {
 	if (T == 0)
 		return hipSuccess;
@@ -1479,17 +1482,15 @@ hipError_t launch_dense(const ExpertTensor &W, const float *x, int T, float *out
 	a.T = T;
 	a.x = x;
 	a.sums[0] = out;
-	a.offsets = ws.offsets;
-	a.pairs = ws.pairs;
-	a.active = ws.active;
 	a.rows = W.rows;
 	a.in = W.in;
 	if (W.type == TIE_GGML_BF16) {
-		tie_launch(dense_groups_kernel, dim3((T + 1 + 255) / 256), dim3(256), 0, s, T, G, ws.offsets, ws.pairs,
-			   ws.active);
+		a.offsets = ws->offsets;
+		a.pairs = ws->pairs;
+		a.active = ws->active;
+		tie_launch(dense_groups_kernel, dim3((T + 1 + 255) / 256), dim3(256), 0, s, T, G, a.offsets, a.pairs, a.active);
 		return launch_gu_bf16(dim3(W.rows / PANEL_ROWS, G, 1), s, a);
 	}
-	a.dense = 1;
 	return launch_gu_q(W.type, false, 1, W.rows, W.in, G, a, s, true);
 }
 
