@@ -63,9 +63,9 @@ struct Ctx {
 	uint32_t *rsq = nullptr;   // host RSQRTSS table (built at the first residual call)
 	int rsq_bits = 0;
 	// TIE_HIP_PATH_AUTO: TIE's bit-exact kernels up to this many tokens,
-	// the matrix cores above (measured faster from T = 22 on at the 30B
-	// shape, graph-timed: T=20 0.1002 / 0.1043 ms, T=22 0.1072 / 0.1065 ms,
-	// T=24 0.1115 / 0.1083 ms exact / MFMA)
+	// the matrix cores above: where they keep within about 6% at the 30B shape
+	// (8 layers, exact / MFMA: T=8 63.1 / 71.8 us, T=12 76.0 / 75.4, T=14 82.2
+	// / 77.4, T=16 87.9 / 83.1, T=20 99.5 / 87.9; 235B T=14 254 / 244)
 	int exact_max_t = 14;
 	int debug_stale = 0; // one-launch decode calls left whose waits are made to give up (debug hook)
 	std::recursive_mutex mu;

@@ -12,13 +12,14 @@
 // more than a launch on this multi-XCD part):
 //   router_small   T <= 4: one workgroup per expert row, row and tokens
 //                  staged in LDS, one thread per (token, lane) chain.
-//   router_mid     2 to 32 tokens (any number when E is not a multiple of
-//                  16): one workgroup per (expert, 16 or 32 tokens), row in
-//                  LDS, x streamed from L2.
+//   router_mid     2 to 32 tokens, and any number where there is no copy of
+//                  the matrix in router_mm's order (E not a multiple of 16;
+//                  F32 matrices of tie_hip_mat_mat): one workgroup per
+//                  (expert, 16 or 32 tokens), row in LDS, x streamed from L2.
 //   router_mm      more: the chains on the fp32 matrix cores.
 // Selection kernel: router_topk (a wave per token, E <= 1024).  Small
-// batches select
-// and group in one workgroup instead (route_group_kernel, dispatch.hip).
+// batches select and group in one workgroup instead (route_group_kernel,
+// dispatch.hip).
 #include "common.h"
 #include "route.h"
 
@@ -251,7 +252,7 @@ router_mm_kernel(const float *__restrict__ x, const float *__restrict__ WM, cons
 	const int net = E / (16 * NE), ntt = (T + TOK - 1) / TOK;
 	int tt, et;
 	if (by_token) {
-		tt = (int)((blockIdx.z * gridDim.y + blockIdx.y) * 8 + blockIdx.x % 8);
+		tt = (int)(blockIdx.y * 8 + blockIdx.x % 8);
 		et = (int)blockIdx.x / 8;
 		if (tt >= ntt)
 			return;
@@ -497,12 +498,10 @@ hipError_t launch_router_logits(const Layer &L, const float *x, int T, float *lo
 			const int by_token = T >= 256 ? 1 : 0; // x the larger operand
 			if (conv)
 				conv->tiles = net;
-			// 8 token tiles x all expert tiles in x, groups of 8 in y and z: one
-			// dimension of tokens times experts would pass the launch limit of 2^32
-			// threads at 2^33 logits (a dense matrix of very many rows)
-			const int n8 = (ntt + 7) / 8, y = n8 < 32768 ? n8 : 32768;
-			tie_launch(kern, by_token ? dim3(8 * net, y, (n8 + y - 1) / y) : dim3(ntt * net), dim3(64 * RM_NW),
-				   0, s, x, L.routerM, L.bias, T, d, E, logits, by_token, z, conv ? *conv : XConvArgs());
+			// 8 token tiles x all expert tiles in x, groups of 8 in y (at most a
+			// 128th of the tokens: the combine has a token in each y)
+			tie_launch(kern, by_token ? dim3(8 * net, (ntt + 7) / 8) : dim3(ntt * net), dim3(64 * RM_NW), 0, s, x,
+				   L.routerM, L.bias, T, d, E, logits, by_token, z, conv ? *conv : XConvArgs());
 		};
 		// larger tiles (fewer x transpositions and weight reads per MFMA) once
 		// they still cover most of the CUs: 30B T=500 (64 tiles of 32 x 32)
