@@ -384,8 +384,8 @@ def test_out_of_range_tokens_recomputed_exactly(seed, E, T, far):
     are recomputed in TIE's exact arithmetic: their rows equal the oracle
     bit for bit, and no other row changes.  E = 16, T = 160: the
     routing kernel converts x and flags the tokens; E = 32, T = 300: the
-    tiled logits kernel does (T > 256), with a flagged token in the last,
-    partial 16-token tile."""
+    matrix-core logits kernel does (T > 256), with a flagged token in the
+    last, partial 16-token tile."""
     layer = synth_layer(seed, 512, 512, E, synth.Q4_K, synth.Q6_K, None)
     k = 4
     x = synth.make_input(seed, T, 512)
@@ -556,7 +556,7 @@ def test_auto_path_threshold():
 
 def test_graph_replays_of_batches():
     """Batched forwards captured in one HIP graph -- the matrix-core path at
-    T = 32 (one work item per expert and slab) and at T = 300 (tiled router
+    T = 32 (one work item per expert and slab) and at T = 300 (matrix-core router
     logits, selection bytes and bucket_plan, one token beyond the f16 range
     recomputed exactly), and the exact path at T = 8 -- replayed four times
     with eager work on the library stream in between: every replay equals

@@ -82,8 +82,8 @@ def test_host_staging(T):
 @pytest.mark.parametrize("T", [1, 6, 40])
 @pytest.mark.parametrize("offset", [0, 1])
 def test_selection_into_callers_buffers(T, offset):
-    """The selection written straight into 16-byte aligned buffers, copied
-    into others."""
+    """The selection in the caller's buffers, 16-byte aligned and not, and
+    nothing beside it."""
     import torch
     d, F, E, k = 512, 256, 16, 4
     layer = synth_layer(421, d, F, E, synth.Q4_K, synth.Q6_K, None)

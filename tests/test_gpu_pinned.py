@@ -25,8 +25,8 @@ def device():
 
 
 # (tokens, path, allocation of the first call on a stream that fails: its
-# workspace is the first).  One token: the status word, the second, or none;
-# more, and the matrix cores: no second one, so the hook stays armed
+# workspace is the first, the one-launch kernel's status word the second; 0:
+# none)
 @pytest.mark.parametrize("T,path,nth", [(1, tie_amd.PATH_EXACT, 2), (1, tie_amd.PATH_EXACT, 0),
                                         (1, tie_amd.PATH_MFMA, 2), (3, tie_amd.PATH_EXACT, 2)])
 @pytest.mark.parametrize("residual", [False, True])

@@ -329,23 +329,14 @@ static int ensure_workspace(hipStream_t s, int T, int k, int d, int F, int E, Wo
 		return rc;
 	carve_workspace((uint8_t *)mem, P, FF, DD, EE, &w);
 	w.alloc = mem;
+	// (without memory to pin, one token takes the other kernels)
+	if (!w.one_status && (w.one_status = (int32_t *)pin_malloc(64)))
+		*w.one_status = 0;
 	// the one-launch decode's words start at sequence 0 (every call uses a
 	// later one)
 	HIP_TRY(hipMemset(w.one_lg, 0, ONE_LG_COPIES * one_copy_words(EE) * 8));
 	HIP_TRY(hipMemset(w.one_h, 0, ONE_H_COPIES * one_copy_words((size_t)MAX_K * FF) * 8));
 	return TIE_HIP_OK;
-}
-
-// The one-launch decode's status word of a workspace, at its first such
-// call; null without memory to pin (the call then takes the other kernels)
-static int32_t *ensure_status(Workspace &w)
-{
-	if (!w.one_status) {
-		w.one_status = (int32_t *)pin_malloc(64);
-		if (w.one_status)
-			*w.one_status = 0;
-	}
-	return w.one_status;
 }
 
 // The status word of stream s's workspace: TIE_HIP_EHIP (and the word
@@ -576,7 +567,7 @@ static int forward(tie_hip_layer *layer, const float *x, int T, int k, float *ou
 	// one token, one launch (eager calls on a workspace of their own: the
 	// sequence number lives on the host, so a captured graph could not
 	// advance it)
-	const bool one = !mfma && T == 1 && !preset && !capturing(s) && decode_one_supported(L, k) && ensure_status(ws);
+	const bool one = !mfma && T == 1 && !preset && !capturing(s) && ws.one_status && decode_one_supported(L, k);
 	if (norm && !(one && decode_one_norm_supported(L, k))) {
 		// (the one-launch kernel normalises its token itself)
 		prof_begin("rmsnorm", s);

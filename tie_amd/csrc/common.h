@@ -141,8 +141,8 @@ struct Workspace {
 	unsigned long long *one_h = nullptr; // [ONE_H_COPIES][MAX_K * F, 4 KiB rows] one-launch decode: {seq, h} words
 	uint32_t one_seq = 0;         // one-launch decode: sequence number of the last call
 	int32_t *one_status = nullptr; // [1] one-launch decode: 1 when a wait gave up (outputs NaN); pinned host
-	                               //     memory, from that kernel's first call on the stream, kept when the
-	                               //     workspace grows
+	                               //     memory, kept when the workspace grows (null: none to be had, or the
+	                               //     no-allocation scratch; that kernel does not run)
 	size_t cap_pairs = 0, cap_F = 0, cap_d = 0, cap_E = 0;
 	void *alloc = nullptr;
 };
