@@ -397,7 +397,7 @@ def cpu_has(flag):
 def cpu_pool_threads():
     """TIE's thread-pool size for the CPU leg: min(nproc, 32), at least k = 8
     (model_qwen3.c:413 indexes tasks[num_threads] by slot), and no more than
-    this process's CPU share (OMP_NUM_THREADS, which the GPU box sets to it)."""
+    this process's CPU share where OMP_NUM_THREADS states it."""
     try:
         nproc = len(os.sched_getaffinity(0))
     except (AttributeError, OSError):
@@ -590,7 +590,7 @@ def main():
         "kernels": m["kernels"],
         "extra": extra,
     }
-    # the two figures BASELINE's metric is quoted on: the 30B block at T=1
+    # the two figures the block's metric is quoted on: the 30B block at T=1
     # (HBM GB/s of its algorithmic bytes) and at T=2048 (MFMA TFLOP/s)
     if "30b_t1" in results:
         line["t1_block_GBps"] = round(results["30b_t1"]["block_GBps"], 1)

@@ -36,7 +36,7 @@ pytestmark = pytest.mark.gpu
 ORACLE_RL2 = 1e-3
 ORACLE_MAXREL = 1e-3
 MODEL_RL2 = 3e-4
-# BF16 weights (activations split into two bf16 parts): the north star's max
+# BF16 weights (activations split into two bf16 parts): the allowed max
 # |err| bound (values O(1)), and rel. L2 (measured 4.4e-6 .. 4.6e-6)
 BF16_MAXABS = 1e-3
 BF16_RL2 = 2e-5

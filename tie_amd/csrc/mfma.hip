@@ -307,10 +307,10 @@ template <int TYPE, bool DOWN = false, int MTR = 0> struct Cfg {
 	// stage, these chunks were a third of Q6_K's L2-to-LDS bytes and a quarter
 	// of Q4_K's.  Kernels, without / with (same weight DMA order, one card):
 	// down Q6_K 30B T=32 35.8 / 33.4 us, T=101 42.4 / 40.2, T=500 52.6 / 49.5,
-	// T=2048 100 / 94, 235B T=1024 202 / 185; gate/up Q4_K 32-row tiles T=32
+	// T=2048 100 / 96, 235B T=1024 202 / 187; gate/up Q4_K 32-row tiles T=32
 	// 42.9 / 41.1, T=64 48.4 / 44.4; Q6_K T=64 63.7 / 62.4; 64-row tiles
 	// Q4_K 30B T=500 65.6 / 67.2 (d = 2048), 235B T=1024 300 / 284, Q6_K
-	// T=500 99 / 89; 160-row tiles Q4_K T=2048 126 / 127, Q6_K 186 / 179 (the
+	// T=500 99 / 89; 160-row tiles Q4_K T=2048 126 / 129, Q6_K 186 / 179 (the
 	// Q6_K 32- and 160-row gate/up kernels are ahead although they spill 1 and
 	// 3 registers with it; Q4_K's 160-row one spills 1 either way).
 	static constexpr bool RES = F16 && KST == 64 && KS == 1 && NS == 2 && QK / KST == 4;

@@ -208,7 +208,7 @@ __global__ __launch_bounds__(TOK * 8) void router_mid_kernel(const float *__rest
 // us at 2048 x 2048 x 128; the kernel without its loads and LDS traffic took
 // 15 us there), else the latency of the launch and the first loads (about 4
 // us) and of the chunks.  Against the kernels it replaced (LDS-tiled vector
-// FMAs above 256 tokens, router_mid below; 30B shape, same box): T=64 7.7 ->
+// FMAs above 256 tokens, router_mid below; 30B shape, same card): T=64 7.7 ->
 // 6.9 us, T=101 11.5 -> 7.3, T=256 19.7 -> 7.0, T=500 17.9 -> 9.3, T=1024
 // 19.4 -> 12.5, T=2048 28.2 -> 19.4; 235B T=1024 35.0 -> 19.6.  Up to 32
 // tokens router_mid stays: T=32 6.3 us against 7.2, T=8 5.0 against 6.5.
